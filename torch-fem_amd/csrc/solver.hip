@@ -18,7 +18,7 @@
 // solution, the residual is replaced by the true FP64 residual b - K x, and
 // the direction is re-orthogonalised against it. Iteration counts therefore
 // stay close to those of FP64 CG, while every iteration streams FP32 values.
-#include "tfm_common.h"
+#include "solver_common.h"
 
 #include <algorithm>
 #include <cmath>
@@ -107,24 +107,6 @@ __device__ __forceinline__ void sum_partials(const double *part, int nblk, doubl
 }
 
 // ------------------------------------------------------- node-block SpMV
-// K contiguous values loaded as one unit (one global_load_dwordxN per lane
-// where the width allows; the compiler otherwise splits rows unevenly).
-template <typename T, int K> struct Vec {
-  T v[K];
-};
-
-template <typename T, int K>
-__device__ __forceinline__ Vec<T, K> ldv(const T *p) {
-  Vec<T, K> r;
-  __builtin_memcpy(&r, p, sizeof(r));
-  return r;
-}
-
-template <typename T, int K>
-__device__ __forceinline__ void stv(T *p, const Vec<T, K> &v) {
-  __builtin_memcpy(p, &v, sizeof(v));
-}
-
 // Neighbour blocks per lane whose loads are issued before any FMA: two for
 // 16-lane FP64 teams (a 27-block Hexa1 row in one pass), one for 32-lane
 // teams and for the FP32 products summed in FP64 (whose wider products
@@ -438,53 +420,11 @@ __global__ void __launch_bounds__(BS) k_spmv_csr(int64_t n, const int64_t *rowpt
 // (Jacobi) in the inner precision; a zero pivot keeps the identity. The
 // inverse is symmetric and stored packed: the upper triangle, row by row,
 // ND*(ND+1)/2 values per node (pc_index).
-template <int ND> constexpr int pc_size() { return ND * (ND + 1) / 2; }
-
-template <int ND>
-__host__ __device__ constexpr int pc_index(int a, int b) {
-  return a <= b ? a * ND - a * (a - 1) / 2 + (b - a) : b * ND - b * (b - 1) / 2 + (a - b);
-}
-
 template <typename T, int ND>
 __global__ void k_precond(int64_t n_nod, const double *dblk, int pc, T *minv) {
   const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= n_nod) return;
-  constexpr int ND2 = ND * ND;
-  double A[ND][ND], R[ND][ND];
-  for (int a = 0; a < ND; ++a)
-    for (int b = 0; b < ND; ++b) {
-      A[a][b] = dblk[n * ND2 + a * ND + b];
-      R[a][b] = a == b ? 1.0 : 0.0;
-    }
-  if (pc == TFM_PC_JACOBI || ND == 1) {
-    for (int a = 0; a < ND; ++a)
-      for (int b = 0; b < ND; ++b) R[a][b] = (a == b && A[a][a] != 0.0) ? 1.0 / A[a][a] : (a == b);
-  } else {
-    // Gauss-Jordan with partial pivoting on the small SPD block
-    for (int c = 0; c < ND; ++c) {
-      int piv = c;
-      for (int r = c + 1; r < ND; ++r)
-        if (fabs(A[r][c]) > fabs(A[piv][c])) piv = r;
-      if (A[piv][c] == 0.0) continue;
-      if (piv != c)
-        for (int k = 0; k < ND; ++k) {
-          double t = A[c][k]; A[c][k] = A[piv][k]; A[piv][k] = t;
-          t = R[c][k]; R[c][k] = R[piv][k]; R[piv][k] = t;
-        }
-      const double inv = 1.0 / A[c][c];
-      for (int k = 0; k < ND; ++k) { A[c][k] *= inv; R[c][k] *= inv; }
-      for (int r = 0; r < ND; ++r)
-        if (r != c) {
-          const double f = A[r][c];
-          for (int k = 0; k < ND; ++k) { A[r][k] -= f * A[c][k]; R[r][k] -= f * R[c][k]; }
-        }
-    }
-  }
-  // the two triangles of the inverse agree up to rounding; their mean keeps
-  // the preconditioner exactly symmetric
-  for (int a = 0; a < ND; ++a)
-    for (int b = a; b < ND; ++b)
-      minv[n * pc_size<ND>() + pc_index<ND>(a, b)] = (T)(0.5 * (R[a][b] + R[b][a]));
+  invert_block<T, ND>(dblk + n * ND * ND, pc, minv + n * pc_size<ND>());
 }
 
 template <typename T, int ND, int NRP>
@@ -1010,15 +950,6 @@ __global__ void k_mask(int64_t n, const uint8_t *con, const double *x, double *x
 // term): the residual then has no FP64 rounding floor of the size
 // eps * |K| |x|, which near a tight tolerance would stall the refinement.
 // One team of TL lanes per node; partials of (res.res, b.b) per block.
-__device__ __forceinline__ void dd_add(double &hi, double &lo, double a, double b2) {
-  // (hi, lo) += (a, b2)
-  const double s = hi + a;
-  const double v = s - hi;
-  const double e = (hi - (s - v)) + (a - v) + lo + b2;
-  hi = s + e;
-  lo = e - (hi - s);
-}
-
 template <int ND, int TL>
 __global__ void __launch_bounds__(BS) k_residual_dd(tfm_mesh_t m, const double *__restrict__ val,
                                                     const double *__restrict__ b,
@@ -1735,6 +1666,9 @@ struct tfm_pcg {
   int *h_done = nullptr;                                   // pinned host mirrors
   double *h_res = nullptr;
   double *h_scal = nullptr;                                // a batch's scalars
+  void *persist = nullptr;                                 // scratch of the persistent solver
+  PersistResult *h_persist = nullptr;                      // its outcome (pinned)
+  bool persist_off = false;  // a persistent solve found the GPU shared (PERSIST_ABORTED)
   // optional event timing of the SpMV launches (kernel A) of the iterations
   // the FP32 arithmetic of the last mixed solve broke down (p.Kp <= 0, or a
   // true residual that stopped falling), and the FP64 iterations that finished it
@@ -1781,6 +1715,8 @@ static int pcg_alloc(tfm_pcg *h) {
   TFM_CHECK_HIP(hipHostMalloc(&h->h_res, sizeof(double) * 4, hipHostMallocDefault));
   TFM_CHECK_HIP(hipHostMalloc(&h->h_scal, sizeof(double) * PCG_CHK_MAX * nrp * NSCAL,
                               hipHostMallocDefault));
+  TFM_CHECK_HIP(hipMalloc(&h->persist, PERSIST_SCRATCH_BYTES));
+  TFM_CHECK_HIP(hipHostMalloc(&h->h_persist, sizeof(PersistResult), hipHostMallocDefault));
   for (auto &e : h->ev) TFM_CHECK_HIP(hipEventCreate(&e));
   return TFM_OK;
 }
@@ -1797,6 +1733,8 @@ static void pcg_free(tfm_pcg *h) {
   if (h->h_done) (void)hipHostFree(h->h_done);
   if (h->h_res) (void)hipHostFree(h->h_res);
   if (h->h_scal) (void)hipHostFree(h->h_scal);
+  if (h->persist) (void)hipFree(h->persist);
+  if (h->h_persist) (void)hipHostFree(h->h_persist);
   for (auto &e : h->ev)
     if (e) (void)hipEventDestroy(e);
 }
@@ -2285,6 +2223,41 @@ int run_pcg(tfm_pcg *h, hipStream_t s, int64_t n_nod, Ops<T> &ops, const double 
   return TFM_OK;
 }
 
+// A system of one rhs that suits the persistent solver: *rc is run_pcg's
+// return value then, and true is returned. Timed solves (tfm_pcg_timing) take
+// the general path, whose launches they time.
+bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, double *relres,
+                 int32_t *outer, int *rc) {
+  if (h->timing || h->persist_off) return false;
+  job.u = h->u;
+  job.p = h->p;
+  job.scratch = h->persist;
+  job.h_res = h->h_persist;
+  job.max_iter = h->max_iter;
+  PersistResult res{};
+  bool ran = false;
+  *rc = persist_solve(s, job, &res, &ran);
+  if (*rc != TFM_OK) return true;
+  if (!ran) {
+    h->persist_off = res.status == PERSIST_ABORTED;
+    return false;
+  }
+  iters[0] = res.iters;
+  relres[0] = res.relres;
+  if (outer) *outer = res.segments;
+  h->breakdown = res.status == PERSIST_NOT_PD || res.status == PERSIST_STAGNATED;
+  if (res.status == PERSIST_OK) return true;
+  *rc = TFM_ERR_NOCONV;
+  set_error(res.status == PERSIST_NOT_PD
+                ? "the matrix is not positive definite (p.Kp <= 0 in CG)"
+            : res.status == PERSIST_STAGNATED
+                ? "PCG stagnated above the tolerance (attainable accuracy reached)"
+            : res.status == PERSIST_NONFINITE
+                ? "non-finite residual in the PCG solve"
+                : "PCG did not reach the tolerance within max_iter iterations");
+  return true;
+}
+
 template <typename T>
 int build_precond(hipStream_t s, int64_t n_nod, int nd, const double *dblk, int pc, T *minv) {
   const unsigned g = (unsigned)((n_nod + 255) / 256);
@@ -2379,7 +2352,26 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
   };
   h->fallback_iters = 0;
   TFM_ND_SWITCH(m.ndof, TFM_NRP_SWITCH(nrp, {
+    auto small = [&](bool fp64, int32_t *its, int32_t *out, int *rcs) -> bool {
+      if (NRP != 1 || cs || !sys->val64) return false;
+      PersistJob job;
+      job.m = &m;
+      job.fp64 = fp64;
+      job.val = fp64 ? (const void *)sys->val64 : (const void *)sys->val32;
+      job.val64 = sys->val64;
+      job.dblk = sys->diag_blocks;
+      job.pc = pc;
+      job.b = b;
+      job.x = x;
+      job.rtol = rtol;
+      job.delta = inner_rtol;
+      job.final_rtol = final_rtol;
+      job.extended = extended;
+      return try_persist(h, s, job, its, relres, out, rcs);
+    };
     auto run_fp64 = [&](int32_t *its, int32_t *out) -> int {
+      int rcs = TFM_OK;
+      if (small(true, its, out, &rcs)) return rcs;
       int rc64 = build_precond<double>(s, m.n_nod, ND, sys->diag_blocks, pc, (double *)h->minv);
       if (rc64 != TFM_OK) return rc64;
       Ops<double> ops;
@@ -2400,22 +2392,24 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
     if (prec == TFM_PREC_FP64) {
       rc = run_fp64(iters, outer);
     } else {
-      rc = build_precond<float>(s, m.n_nod, ND, sys->diag_blocks, pc, (float *)h->minv);
-      if (rc != TFM_OK) return rc;
-      Ops<float> ops;
-      ops.scal = spmv_shape<float>(m, NRP).scal;
-      ops.spmv_dir = [&](const float *u, float *p, float *sv, int it, const double *pin,
-                         int n_in, const PcgState &st, unsigned *g) -> int {
-        return spmv_dir_launch<float, ND, NRP>(s, m, sys->val32, u, p, sv, it, pin, n_in, st,
-                                               g);
-      };
-      ops.spmv = [&](const float *xi, float *yo) -> int {
-        return spmv_launch<float, ND, NRP>(s, m, sys->val32, xi, yo);
-      };
-      ops.residual = residual;
-      if (cs) ops.coarse = coarse_ops<float, ND, NRP>(s, m, *cs, sys->con, cs->inv32);
-      rc = run_pcg<float, ND, NRP>(h, s, m.n_nod, ops, b, x, nrhs, rtol, inner_rtol, final_rtol,
-                                   iters, relres, outer);
+      if (!small(false, iters, outer, &rc)) {
+        rc = build_precond<float>(s, m.n_nod, ND, sys->diag_blocks, pc, (float *)h->minv);
+        if (rc != TFM_OK) return rc;
+        Ops<float> ops;
+        ops.scal = spmv_shape<float>(m, NRP).scal;
+        ops.spmv_dir = [&](const float *u, float *p, float *sv, int it, const double *pin,
+                           int n_in, const PcgState &st, unsigned *g) -> int {
+          return spmv_dir_launch<float, ND, NRP>(s, m, sys->val32, u, p, sv, it, pin, n_in, st,
+                                                 g);
+        };
+        ops.spmv = [&](const float *xi, float *yo) -> int {
+          return spmv_launch<float, ND, NRP>(s, m, sys->val32, xi, yo);
+        };
+        ops.residual = residual;
+        if (cs) ops.coarse = coarse_ops<float, ND, NRP>(s, m, *cs, sys->con, cs->inv32);
+        rc = run_pcg<float, ND, NRP>(h, s, m.n_nod, ops, b, x, nrhs, rtol, inner_rtol, final_rtol,
+                                     iters, relres, outer);
+      }
       // FP32 rounding of a matrix whose element stiffnesses span many orders
       // of magnitude (void elements of a density design) can make the FP32
       // operator indefinite or cap the accuracy of its corrections: then
@@ -2477,6 +2471,20 @@ extern "C" int tfm_csr_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, int64_t n,
   TFM_REQUIRE(n == h->n, "system size differs from the solver handle");
   TFM_REQUIRE(rtol > 0.0, "rtol must be positive");
   hipStream_t s = (hipStream_t)stream;
+  {
+    PersistJob job;
+    job.n = n;
+    job.rowptr = rowptr;
+    job.col = col;
+    job.val = val;
+    job.val64 = val;
+    job.b = b;
+    job.x = x;
+    job.rtol = rtol;
+    job.final_rtol = 0.7 * rtol;
+    int rc = TFM_OK;
+    if (try_persist(h, s, job, iters, relres, nullptr, &rc)) return rc;
+  }
   const unsigned g1 = (unsigned)((n + 255) / 256);
   hipLaunchKernelGGL(k_csr_diag, dim3(g1), dim3(256), 0, s, n, rowptr, col, val, h->f64);
   TFM_CHECK_LAUNCH();
