@@ -35,7 +35,6 @@ constexpr int RBA = 2048; // max blocks of the SpMV kernels (= eta partials per 
 constexpr int RBV = 512;  // max blocks of the vector kernels whose partials every block of A sums
 constexpr int RBW = 4096; // max blocks of the vector kernels when a scalar kernel sums them
 constexpr int MAXR = 16;  // right-hand sides per solve
-constexpr int CGB = 1;    // partial sets of the coarse correction (after the update's)
 constexpr int NSCAL = 4;  // per-iteration scalars: rz, pq, rr, spare
 constexpr int PCG_CHK_MAX = 64;  // most iterations between two host checks
 enum { S_RZ = 0, S_PQ = 1, S_RR = 2 };
@@ -72,25 +71,31 @@ __device__ __forceinline__ void write_block_partials(const double (&v)[NV], doub
 
 // Sums the NVT partial slots written by nblk blocks into out[0..NVT) in LDS,
 // in a fixed order, so that every block that calls it gets the same bits.
-// Thread t adds the partials b = t/NVT + k*CH of slot t % NVT with four
-// loads in flight; a wave butterfly and one LDS stage over the waves follow
-// (one thread adding a 256-long LDS column serially costs microseconds).
+// Thread t adds the partials b = t/NVT + k*CH of slot t % NVT, eight loads in
+// flight (loads past the end read the last set again and count as zero: a
+// bounds test per load would make each wait for the one before); a wave
+// butterfly and one LDS stage over the waves follow (one thread adding a
+// 256-long LDS column serially costs microseconds).
 template <int NVT, int BSZ = BS>
 __device__ __forceinline__ void sum_partials(const double *part, int nblk, double *sh,
                                              double *out) {
   static_assert(64 % NVT == 0 && BSZ % 64 == 0, "slots must tile a wave");
-  constexpr int CH = BSZ / NVT, NW = BSZ / 64;
+  constexpr int CH = BSZ / NVT, NW = BSZ / 64, U = 8;
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int slot = tid % NVT;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  int b = tid / NVT;
-  for (; b + 3 * CH < nblk; b += 4 * CH) {
-    a0 += part[(size_t)b * NVT + slot];
-    a1 += part[(size_t)(b + CH) * NVT + slot];
-    a2 += part[(size_t)(b + 2 * CH) * NVT + slot];
-    a3 += part[(size_t)(b + 3 * CH) * NVT + slot];
+  for (int b = tid / NVT; b < nblk; b += U * CH) {
+    double v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = part[(size_t)min(b + k * CH, nblk - 1) * NVT + slot];
+#pragma unroll
+    for (int k = 1; k < U; ++k)
+      if (b + k * CH >= nblk) v[k] = 0.0;
+    a0 += v[0] + v[4];
+    a1 += v[1] + v[5];
+    a2 += v[2] + v[6];
+    a3 += v[3] + v[7];
   }
-  for (; b < nblk; b += CH) a0 += part[(size_t)b * NVT + slot];
   double acc = (a0 + a1) + (a2 + a3);
 #pragma unroll
   for (int off = NVT; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
@@ -870,12 +875,13 @@ __global__ void __launch_bounds__(BS) k_pcg_seg_dots(int64_t n_nod, const T *r, 
 template <typename T, int ND, int NRP>
 __global__ void __launch_bounds__(BS) k_pcg_seg_apply(int64_t n_nod, int it, int mask, int cont,
                                                       int running, SegInfo seg, const T *u, T *p,
-                                                      T *s, PcgState st, int nblk, int nblk_aux) {
+                                                      T *s, PcgState st, const double *sets,
+                                                      int nblk, const double *aux, int nblk_aux) {
   __shared__ double sh[BS];
   __shared__ double tot[2 * NRP], rp[NRP], cz[NRP];
   __shared__ int mode[NRP];
-  sum_partials<2 * NRP>(st.part_upd, nblk, sh, tot);
-  sum_partials<NRP>(st.part_aux, nblk_aux, sh, rp);
+  sum_partials<2 * NRP>(sets, nblk, sh, tot);
+  sum_partials<NRP>(aux, nblk_aux, sh, rp);
   const int tid = threadIdx.x;
   if (tid < NRP) {
     const bool run = (mask >> tid) & 1;
@@ -1283,7 +1289,10 @@ struct CoarseView {
   int n_agg, n_c;
   const int32_t *agg, *agg_ptr, *agg_nodes, *slot_agg, *pair_off, *pair_node, *pair_pos;
   const double *cen;
-  double *rc, *ec;  // [n_c * NRP]
+  double *rc;    // [chunks][n_c][NRP] restricted residual, one part per chunk
+  double *part;  // partial sets of the update, then those of the coarse correction
+  double *aux;   // r.p partials of a segment start
+  int *never;    // a flag that stays 0
 };
 
 // Ac[(I nm + k), (J nm + l)] for the aggregate pair (I, slot): one wave per
@@ -1338,124 +1347,324 @@ __global__ void __launch_bounds__(64) k_coarse_operator(tfm_mesh_t m, CoarseView
   }
 }
 
-// Sums of v over the lanes of each wave that share lane % NRP (a butterfly
-// in a fixed order), then over the block's waves in wave order, for the
-// values of one block of NT threads; the result is valid in threads
-// 0 .. NRP - 1 (rhs = thread). Every thread of the block must call it.
-template <int NRP, int NT = BS>
-__device__ __forceinline__ double block_sum_by_rhs(double v, double *sh) {
-  for (int off = 32; off >= NRP; off >>= 1) v += __shfl_xor(v, off, 64);
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  if (lane < NRP) sh[wave * NRP + lane] = v;
-  __syncthreads();
-  double tsum = 0.0;
-  if (threadIdx.x < NRP)
-    for (int w = 0; w < NT / 64; ++w) tsum += sh[w * NRP + threadIdx.x];
-  __syncthreads();
-  return tsum;
+// Work of the two fused kernels below. The update takes a block per chunk of
+// an aggregate's nodes, the coarse product a block per chunk as well, or, for
+// scalar fields, whose aggregates have one mode, one per four aggregates.
+// With one or two right-hand sides a block has 256 threads and a chunk at most
+// about 256 nodes (one per thread); with four or more it has 1024, which the
+// NRP entries of a chunk's nodes fill several times.
+template <int ND, int NRP> struct CoarseShape {
+  static constexpr int THREADS = NRP >= 4 ? 1024 : 256;
+  static constexpr int WAVES = THREADS / 64;
+  static constexpr int AGGS = ND == 1 && NRP <= 2 ? 4 : 1;  // per block of the coarse product
+  static int chunks(int64_t n_nod, int n_agg) {
+    const int64_t per = (n_nod + n_agg - 1) / n_agg;
+    if (AGGS > 1) return 1;
+    if (NRP >= 4) return 1;  // two chunks: 27.0 + 20.2 us, not 15.0 + 16.6 (Hexa2 21 x 19 x 23)
+    return per > 512 ? 4 : per > 256 ? 2 : 1;
+  }
+};
+
+// Sum over the lanes of a wave with the same lane % NRP, valid in every lane.
+template <int NRP> __device__ __forceinline__ double rhs_lanes_sum(double v) {
+  if constexpr (NRP == 1) return lanes_sum<64>(v);
+  for (int off = NRP; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+  return butterfly_partner_sum<32>(butterfly_partner_sum<16>(v));
 }
 
-// r_c = P^T r: one block per aggregate; thread t takes rhs t % NRP of every
-// (BS / NRP)-th node of the aggregate, and the block adds the thread sums by
-// waves (block_sum_by_rhs). (Blocks of 1024 threads, one node per thread,
-// measured slower: 11.2 against 8.9 us on the 64^3 cube.)
-template <typename T, int ND, int NRP>
-__global__ void __launch_bounds__(BS) k_coarse_restrict(tfm_mesh_t m, CoarseView cv,
-                                                        const uint8_t *con, const T *r,
-                                                        const int *alldone) {
-  constexpr int NM = coarse_modes<ND>(), CH = BS / NRP;
-  __shared__ double sh[BS / 64 * NRP];
-  if (*alldone) return;
-  const int I = blockIdx.x, t = threadIdx.x, rr = t % NRP, c = t / NRP;
-  double acc[NM];
-  for (int k = 0; k < NM; ++k) acc[k] = 0.0;
-  for (int q = cv.agg_ptr[I] + c; q < cv.agg_ptr[I + 1]; q += CH) {
-    const int64_t i = cv.agg_nodes[q];
-    double M[ND][NM];
-    node_modes<ND>(m, cv.cen, con, i, I, M);
+// The nodes [q0, q1) of agg_nodes in chunk c of aggregate I.
+__device__ __forceinline__ void unit_nodes(const CoarseView &cv, int I, int c, int chunks,
+                                           int &q0, int &q1) {
+  const int beg = cv.agg_ptr[I], len = cv.agg_ptr[I + 1] - beg;
+  q0 = beg + (int)((int64_t)len * c / chunks);
+  q1 = beg + (int)((int64_t)len * (c + 1) / chunks);
+}
+
+// B with the restriction of the coarse correction, over the nodes of the
+// aggregates: alpha = gamma / eta; x += alpha p; r -= alpha s; u = B^{-1} r;
+// partials of (r.u, r.r); and this chunk's part of r_c = P^T r. SEG: the
+// start of a segment instead (no update; partials of r.p as well).
+// One launch in the place of two: the restriction read r again and spent its
+// time on the chain aggregate -> node -> coordinates, which the update now
+// hides (6.7 + 5.6 us on the 47 x 41 x 52 cube before).
+template <typename T, int ND, int NRP, bool CO, bool SEG>
+__global__ void __launch_bounds__((CoarseShape<ND, NRP>::THREADS))
+k_pcg_update_restrict(tfm_mesh_t m, CoarseView cv, const uint8_t *__restrict__ con, int chunks,
+                      int it, T *__restrict__ x, T *__restrict__ r, T *__restrict__ u,
+                      const T *__restrict__ p, const T *__restrict__ s,
+                      const T *__restrict__ minv, PcgState st, const double *pq_in, int n_pq) {
+  using Shape = CoarseShape<ND, NRP>;
+  constexpr int NM = coarse_modes<ND>(), NT = Shape::THREADS, NW = Shape::WAVES;
+  constexpr int NV = 2 + (SEG ? 1 : 0);
+  __shared__ double sh[NW * (NV + NM) * NRP > NT ? NW * (NV + NM) * NRP : NT];
+  __shared__ double pq[NRP], alpha[NRP];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int blk = (int)xcd_block();
+  const int I = blk / chunks, c = blk % chunks;
+  int q0, q1;
+  unit_nodes(cv, I, c, chunks, q0, q1);
+  constexpr int STEP = NT / NRP;
+  const int rr = tid % NRP;
+  int q = q0 + tid / NRP;
+  int64_t n = 0;
+  Vec<T, pc_size<ND>()> mi;
+  T xv[ND], rv[ND], pv[ND], sv[ND];
+  double d[ND];
+  int free_mask = 0;
+  auto load = [&]() {
+    n = cv.agg_nodes[q];
+    mi = ldv<T, pc_size<ND>()>(minv + n * pc_size<ND>());
+#pragma unroll
     for (int a = 0; a < ND; ++a) {
-      const double rv = (double)r[(i * ND + a) * NRP + rr];
-      for (int k = 0; k < NM; ++k) acc[k] += M[a][k] * rv;
+      const int64_t o = (n * ND + a) * NRP + rr;
+      rv[a] = r[o];
+      pv[a] = p[o];
+      if constexpr (!SEG) {
+        xv[a] = x[o];
+        sv[a] = s[o];
+      }
+      if constexpr (ND > 1) d[a] = m.nodes[n * ND + a];
     }
+    free_mask = 0;
+#pragma unroll
+    for (int a = 0; a < ND; ++a) free_mask |= con[n * ND + a] ? 0 : 1 << a;
+  };
+  if constexpr (SEG) {
+    if (q < q1) load();
+  } else if constexpr (CO) {  // alpha prepared by k_pcg_scal_alpha
+    const PcgCoef &cf = *st.coef_b;
+    if (!cf.any) return;
+    if (q < q1) load();
+    if (tid < NRP) alpha[tid] = cf.c[tid];
+    __syncthreads();
+  } else {
+    const int ended = *st.alldone;  // tested after the sums, so the loads overlap
+    if (q < q1) load();
+    sum_partials<NRP, NT>(pq_in, n_pq, sh, pq);
+    if (ended) return;
+    if (tid < NRP) {
+      double *sc = st.scal + ((size_t)it * NRP + tid) * NSCAL;
+      alpha[tid] = (st.done[tid] < 0 && pq[tid] != 0.0) ? sc[S_RZ] / pq[tid] : 0.0;
+      if (blk == 0) sc[S_PQ] = pq[tid];
+    }
+    __syncthreads();
   }
-  for (int k = 0; k < NM; ++k) {
-    const double v = block_sum_by_rhs<NRP>(acc[k], sh);
-    if (t < NRP) cv.rc[((int64_t)I * NM + k) * NRP + t] = v;
+  double cen[ND];
+  if constexpr (ND > 1)
+    for (int a = 0; a < ND; ++a) cen[a] = cv.cen[(int64_t)I * ND + a];
+  double v[NV + NM];
+#pragma unroll
+  for (int k = 0; k < NV + NM; ++k) v[k] = 0.0;
+  T al = T(0);
+  if constexpr (!SEG) al = (T)alpha[rr];
+  while (q < q1) {
+    T zv[ND];
+    if constexpr (!SEG) {
+#pragma unroll
+      for (int a = 0; a < ND; ++a) {
+        xv[a] += al * pv[a];
+        rv[a] -= al * sv[a];
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+      T z = T(0);
+#pragma unroll
+      for (int b = 0; b < ND; ++b) z += mi.v[pc_index<ND>(a, b)] * rv[b];
+      zv[a] = z;
+      v[0] += (double)rv[a] * (double)z;
+      v[1] += (double)rv[a] * (double)rv[a];
+      if constexpr (SEG) v[2] += (double)rv[a] * (double)pv[a];
+    }
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+      const int64_t o = (n * ND + a) * NRP + rr;
+      u[o] = zv[a];
+      if constexpr (!SEG) {
+        x[o] = xv[a];
+        r[o] = rv[a];
+      }
+    }
+    // P^T r: translations, then the rotations e_k x d about the centroid
+    double f[ND];
+#pragma unroll
+    for (int a = 0; a < ND; ++a) f[a] = (free_mask >> a) & 1 ? (double)rv[a] : 0.0;
+#pragma unroll
+    for (int a = 0; a < ND; ++a) v[NV + a] += f[a];
+    if constexpr (ND == 3) {
+#pragma unroll
+      for (int a = 0; a < ND; ++a) d[a] -= cen[a];
+      v[NV + 3] += d[1] * f[2] - d[2] * f[1];
+      v[NV + 4] += d[2] * f[0] - d[0] * f[2];
+      v[NV + 5] += d[0] * f[1] - d[1] * f[0];
+    } else if constexpr (ND == 2) {
+#pragma unroll
+      for (int a = 0; a < ND; ++a) d[a] -= cen[a];
+      v[NV + 2] += d[0] * f[1] - d[1] * f[0];
+    }
+    q += STEP;
+    if (q < q1) load();
   }
-}
-
-// e_c = Ainv r_c, one wave per row (four rows per block), columns split
-// over the lanes with four loads in flight, and the lane sums added by a
-// butterfly.
-template <typename TI, int NRP>
-__global__ void __launch_bounds__(BS) k_coarse_solve(CoarseView cv, const TI *inv,
-                                                     const int *alldone) {
-  if (*alldone) return;
-  const int lane = threadIdx.x % 64;
-  const int row = blockIdx.x * (BS / 64) + threadIdx.x / 64;
-  if (row >= cv.n_c) return;
-  double acc[NRP];
-  for (int r = 0; r < NRP; ++r) acc[r] = 0.0;
-  const TI *ar = inv + (int64_t)row * cv.n_c;
-  int col = lane;
-  for (; col + 192 < cv.n_c; col += 256) {
-    const double a0 = (double)ar[col], a1 = (double)ar[col + 64];
-    const double a2 = (double)ar[col + 128], a3 = (double)ar[col + 192];
-    for (int r = 0; r < NRP; ++r)
-      acc[r] += a0 * cv.rc[(int64_t)col * NRP + r] + a1 * cv.rc[(int64_t)(col + 64) * NRP + r] +
-                a2 * cv.rc[(int64_t)(col + 128) * NRP + r] +
-                a3 * cv.rc[(int64_t)(col + 192) * NRP + r];
-  }
-  for (; col < cv.n_c; col += 64) {
-    const double a = (double)ar[col];
-    for (int r = 0; r < NRP; ++r) acc[r] += a * cv.rc[(int64_t)col * NRP + r];
-  }
-  for (int off = 32; off >= 1; off >>= 1)
-    for (int r = 0; r < NRP; ++r) acc[r] += __shfl_xor(acc[r], off, 64);
+#pragma unroll
+  for (int k = 0; k < NV + NM; ++k) v[k] = rhs_lanes_sum<NRP>(v[k]);
+  __syncthreads();  // sh may still be read by sum_partials
   if (lane < NRP) {
-    double e = 0.0;
-    for (int r = 0; r < NRP; ++r)
-      if (r == lane) e = acc[r];
-    cv.ec[(int64_t)row * NRP + lane] = e;
+#pragma unroll
+    for (int k = 0; k < NV + NM; ++k) sh[(wave * (NV + NM) + k) * NRP + lane] = v[k];
+  }
+  __syncthreads();
+  constexpr int NO = (NV + NM) * NRP;
+  if (tid < NO) {
+    const int k = tid / NRP, rr2 = tid % NRP;
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += sh[(w * (NV + NM) + k) * NRP + rr2];
+    if (k < 2) cv.part[((int64_t)blk * 2 + k) * NRP + rr2] = t;
+    else if (k < NV) cv.aux[(int64_t)blk * NRP + rr2] = t;
+    else cv.rc[((int64_t)c * cv.n_c + (int64_t)I * NM + (k - NV)) * NRP + rr2] = t;
   }
 }
 
-// u += P e_c, one thread per (node, rhs). Block 0 also writes r_c . e_c
-// per rhs as one partial set in the (gamma, rr) layout of the PCG's update
-// partials (rr slot 0), summed in a fixed order (block_sum_by_rhs).
-template <typename T, int ND, int NRP>
-__global__ void __launch_bounds__(256) k_coarse_prolong(tfm_mesh_t m, CoarseView cv,
-                                                        const uint8_t *con, T *u, double *part,
-                                                        const int *alldone) {
-  constexpr int NM = coarse_modes<ND>();
-  static_assert(BS == 256, "k_coarse_prolong runs blocks of BS = 256 threads");
-  __shared__ double sh[BS / 64 * NRP];
-  if (*alldone) return;
-  if (blockIdx.x == 0) {
-    const int rr = threadIdx.x % NRP, c = threadIdx.x / NRP;
-    double d = 0.0;
-    for (int row = c; row < cv.n_c; row += BS / NRP)
-      d += cv.rc[(int64_t)row * NRP + rr] * cv.ec[(int64_t)row * NRP + rr];
-    const double t2 = block_sum_by_rhs<NRP>(d, sh);
-    if (threadIdx.x < NRP) {
-      part[threadIdx.x] = t2;
-      part[NRP + threadIdx.x] = 0.0;
+// The rest of the coarse correction: a block forms its aggregates' rows of
+// e_c = Ainv r_c (R rows at once, the columns split over its threads, r_c
+// summed over the chunks) and adds P e_c to u at its nodes; the first chunk's
+// block writes r_c . e_c of its rows. One more block adds the update's
+// partial sets, so that the next kernel A reads that sum and one set per
+// block with rows. One launch in the place of two: a chunk repeats its
+// aggregate's rows, 6 n_c values from L2, which is less than a launch. Bound
+// by its chain of loads: CB columns are in flight per thread, which is all of
+// them up to 2,048 coarse unknowns, and the first node's entries are loaded
+// ahead of the product (11.1 us on the 47 x 41 x 52 cube with four columns in
+// flight and the nodes loaded after it).
+template <typename T, int ND, int NRP, int CHUNKS>
+__global__ void __launch_bounds__((CoarseShape<ND, NRP>::THREADS))
+k_coarse_apply(tfm_mesh_t m, CoarseView cv, const uint8_t *__restrict__ con,
+               const T *__restrict__ inv, T *__restrict__ u, int n_sets, double *out,
+               const int *flag) {
+  using Shape = CoarseShape<ND, NRP>;
+  constexpr int NM = coarse_modes<ND>(), NT = Shape::THREADS, NW = Shape::WAVES;
+  constexpr int AG = Shape::AGGS;  // aggregates of the block
+  constexpr int R = NM * AG;
+  constexpr int CB = NRP >= 4 || CHUNKS > 2 ? 4 : 8;
+  __shared__ double sh[NW * R * NRP > NT ? NW * R * NRP : NT];
+  __shared__ double e_sh[R * NRP], tot[2 * NRP];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int blk = (int)xcd_block();
+  const int stop = *flag;
+  if (blk == (int)gridDim.x - 1) {
+    if (stop) return;
+    sum_partials<2 * NRP, NT>(cv.part, n_sets, sh, tot);
+    if (tid < 2 * NRP) out[tid] = tot[tid];
+    return;
+  }
+  const int I = AG > 1 ? blk * AG : blk / CHUNKS;
+  const int c = AG > 1 ? 0 : blk % CHUNKS;
+  int q0, q1;
+  if constexpr (AG > 1) {
+    q0 = cv.agg_ptr[I];
+    q1 = cv.agg_ptr[min(I + AG, cv.n_agg)];
+  } else {
+    unit_nodes(cv, I, c, CHUNKS, q0, q1);
+  }
+  constexpr int STEP = NT / NRP;
+  const int rr = tid % NRP, t0 = tid / NRP;
+  // the first node's entries
+  int q = q0 + t0, ag = 0;
+  int64_t n = 0;
+  double d[ND], uo[ND];
+  int free_mask = 0;
+  auto load = [&]() {
+    n = cv.agg_nodes[q];
+    free_mask = 0;
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+      if constexpr (ND > 1) d[a] = m.nodes[n * ND + a];
+      uo[a] = (double)u[(n * ND + a) * NRP + rr];
+      free_mask |= con[n * ND + a] ? 0 : 1 << a;
+    }
+    if constexpr (AG > 1) ag = cv.agg[n] - I;
+  };
+  if (q < q1) load();
+  double cen[ND];
+  if constexpr (ND > 1)
+    for (int a = 0; a < ND; ++a) cen[a] = cv.cen[(int64_t)I * ND + a];
+  if (stop) return;
+  // rows I NM ... of Ainv times r_c
+  const int nc = cv.n_c, rows = min(R, nc - I * NM);
+  const T *ar = inv + (int64_t)I * NM * nc;
+  double e[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) e[k] = 0.0;
+  // Loads beyond the last column read it again and are multiplied by zero: a
+  // bounds test per load made each a branch of its own (19 us, not 8).
+  for (int c0 = t0; c0 < nc; c0 += CB * STEP) {
+    double rv[CHUNKS][CB];
+    T av[CB][R];
+#pragma unroll
+    for (int h = 0; h < CB; ++h) {
+      const int col = min(c0 + h * STEP, nc - 1);
+#pragma unroll
+      for (int g = 0; g < CHUNKS; ++g) rv[g][h] = cv.rc[((int64_t)g * nc + col) * NRP + rr];
+#pragma unroll
+      for (int k = 0; k < R; ++k) av[h][k] = ar[(int64_t)min(k, rows - 1) * nc + col];
+    }
+#pragma unroll
+    for (int h = 0; h < CB; ++h) {
+      double v = rv[0][h];
+#pragma unroll
+      for (int g = 1; g < CHUNKS; ++g) v += rv[g][h];
+      if (c0 + h * STEP >= nc) v = 0.0;
+#pragma unroll
+      for (int k = 0; k < R; ++k) e[k] += (double)av[h][k] * v;
     }
   }
-  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= m.n_nod * NRP) return;
-  const int64_t i = t / NRP;
-  const int rr = (int)(t % NRP);
-  const int I = cv.agg[i];
-  double M[ND][NM];
-  node_modes<ND>(m, cv.cen, con, i, I, M);
-  double e[NM];
-  for (int k = 0; k < NM; ++k) e[k] = cv.ec[((int64_t)I * NM + k) * NRP + rr];
-  for (int a = 0; a < ND; ++a) {
-    double v = 0.0;
-    for (int k = 0; k < NM; ++k) v += M[a][k] * e[k];
-    T *ua = u + (i * ND + a) * NRP + rr;
-    *ua = (T)((double)*ua + v);
+#pragma unroll
+  for (int k = 0; k < R; ++k) e[k] = rhs_lanes_sum<NRP>(e[k]);
+  if (lane < NRP)
+#pragma unroll
+    for (int k = 0; k < R; ++k) sh[(wave * R + k) * NRP + lane] = e[k];
+  __syncthreads();
+  if (tid < R * NRP) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += sh[w * R * NRP + tid];
+    e_sh[tid] = t;
+  }
+  __syncthreads();
+  if (c == 0 && tid < NRP) {  // r_c . e_c of the block's rows
+    double dot = 0.0;
+    for (int k = 0; k < rows; ++k) {
+      double v = 0.0;
+#pragma unroll
+      for (int g = 0; g < CHUNKS; ++g) v += cv.rc[((int64_t)g * nc + I * NM + k) * NRP + tid];
+      dot += v * e_sh[k * NRP + tid];
+    }
+    const int64_t set = 1 + (AG > 1 ? blk : I);
+    out[set * 2 * NRP + tid] = dot;
+    out[(set * 2 + 1) * NRP + tid] = 0.0;
+  }
+  while (q < q1) {
+    double g[ND], ek[NM];
+#pragma unroll
+    for (int k = 0; k < NM; ++k) ek[k] = e_sh[(ag * NM + k) * NRP + rr];
+    if constexpr (ND > 1)
+#pragma unroll
+      for (int a = 0; a < ND; ++a) d[a] -= cen[a];
+    if constexpr (ND == 3) {
+      g[0] = ek[0] + d[2] * ek[4] - d[1] * ek[5];
+      g[1] = ek[1] + d[0] * ek[5] - d[2] * ek[3];
+      g[2] = ek[2] + d[1] * ek[3] - d[0] * ek[4];
+    } else if constexpr (ND == 2) {
+      g[0] = ek[0] - d[1] * ek[2];
+      g[1] = ek[1] + d[0] * ek[2];
+    } else {
+      g[0] = ek[0];
+    }
+#pragma unroll
+    for (int a = 0; a < ND; ++a)
+      if ((free_mask >> a) & 1) u[(n * ND + a) * NRP + rr] = (T)(uo[a] + g[a]);
+    q += STEP;
+    if (q < q1) load();
   }
 }
 
@@ -1625,20 +1834,21 @@ struct tfm_coarse {
   int32_t *agg = nullptr, *agg_ptr = nullptr, *agg_nodes = nullptr, *slot_agg = nullptr;
   int32_t *pair_off = nullptr, *pair_node = nullptr, *pair_pos = nullptr;
   double *cen = nullptr;
-  double *rc = nullptr, *ec = nullptr;  // [n_c * MAXR]
+  double *rc = nullptr;                 // [4 chunks][n_c * MAXR]
+  double *part = nullptr, *aux = nullptr;  // partial sets (CoarseView)
   int *never = nullptr;                 // a device flag that stays 0 (segment starts)
   const double *inv64 = nullptr;        // the caller's inverse of P^T K P
   const float *inv32 = nullptr;
   CoarseView view() const {
     return CoarseView{n_agg, n_c, agg, agg_ptr, agg_nodes, slot_agg, pair_off, pair_node,
-                      pair_pos, cen, rc, ec};
+                      pair_pos, cen, rc, part, aux, never};
   }
 };
 
 static void coarse_free(tfm_coarse *h) {
   for (void *ptr : {(void *)h->agg, (void *)h->agg_ptr, (void *)h->agg_nodes, (void *)h->slot_agg,
                     (void *)h->pair_off, (void *)h->pair_node, (void *)h->pair_pos,
-                    (void *)h->cen, (void *)h->rc, (void *)h->ec, (void *)h->never})
+                    (void *)h->cen, (void *)h->rc, (void *)h->part, (void *)h->aux, (void *)h->never})
     if (ptr) (void)hipFree(ptr);
 }
 
@@ -1702,7 +1912,7 @@ static int pcg_alloc(tfm_pcg *h) {
   // (the 64-lane team), n / 4 covers it for one DOF per node
   h->pq_cap = (int)std::max<int64_t>(RBA, n / 4 + 1);
   TFM_CHECK_HIP(hipMalloc(&h->part_pq, sizeof(double) * (size_t)h->pq_cap * nrp));
-  TFM_CHECK_HIP(hipMalloc(&h->part_upd, sizeof(double) * (RBW + CGB) * 2 * nrp));
+  TFM_CHECK_HIP(hipMalloc(&h->part_upd, sizeof(double) * RBW * 2 * nrp));
   TFM_CHECK_HIP(hipMalloc(&h->part_aux, sizeof(double) * RBW * nrp));
   h->res_cap = (int)std::max<int64_t>(RBV, n / 8 + 1);  // >= n_nod / 8 node teams
   TFM_CHECK_HIP(hipMalloc(&h->part_res, sizeof(double) * (size_t)h->res_cap * 2));
@@ -1812,8 +2022,11 @@ extern "C" int tfm_coarse_create(tfm_coarse_t **out, const tfm_mesh_t *m, int32_
   if (rc == TFM_OK) rc = copy(&h->pair_off, pair_off, (size_t)n_agg * 27 + 1);
   if (rc == TFM_OK) rc = copy(&h->pair_node, pair_node, (size_t)n_pairs);
   if (rc == TFM_OK) rc = copy(&h->pair_pos, pair_pos, (size_t)n_pairs);
-  if (rc == TFM_OK && hipMalloc(&h->rc, sizeof(double) * h->n_c * MAXR) != hipSuccess) rc = TFM_ERR_HIP;
-  if (rc == TFM_OK && hipMalloc(&h->ec, sizeof(double) * h->n_c * MAXR) != hipSuccess) rc = TFM_ERR_HIP;
+  // at most 4 chunks per aggregate: 4 n_agg update sets, n_agg + 1 coarse sets
+  const size_t sets = (size_t)n_agg * 5 + 1;
+  if (rc == TFM_OK && hipMalloc(&h->rc, sizeof(double) * h->n_c * MAXR * 4) != hipSuccess) rc = TFM_ERR_HIP;
+  if (rc == TFM_OK && hipMalloc(&h->part, sizeof(double) * sets * 2 * MAXR) != hipSuccess) rc = TFM_ERR_HIP;
+  if (rc == TFM_OK && hipMalloc(&h->aux, sizeof(double) * n_agg * 4 * MAXR) != hipSuccess) rc = TFM_ERR_HIP;
   if (rc == TFM_OK && hipMalloc(&h->never, sizeof(int)) != hipSuccess) rc = TFM_ERR_HIP;
   if (rc == TFM_OK && hipMemset(h->never, 0, sizeof(int)) != hipSuccess) rc = TFM_ERR_HIP;
   if (rc != TFM_OK) {
@@ -1925,31 +2138,58 @@ template <typename T> struct Ops {
       spmv_dir;
   std::function<int(const T *, T *)> spmv;
   std::function<int(const double *, const double *, double *, double *, double *)> residual;
-  // two-level preconditioner: u += P Ac^{-1} P^T r and the partial sets of
-  // (P^T r).(Ac^{-1} P^T r) at `part`; skipped once *flag is set (empty if unused)
-  std::function<int(const T *, T *, double *, const int *)> coarse;
+  // two-level preconditioner: the update of iteration `it` (or, with it < 0,
+  // the start of a segment) including the coarse correction of u; its
+  // `n_sets` partial sets are at `sets`, its r.p partials (segment start) are
+  // `n_aux` values per rhs at `aux`. Empty without a coarse space.
+  std::function<int(int, T *, T *, T *, const T *, const T *, const T *, const PcgState &,
+                    const double *, int)>
+      update_coarse;
+  double *sets = nullptr, *aux = nullptr;
+  int n_sets = 0, n_aux = 0;
 };
 
-// The coarse correction's three launches: r_c = P^T r, e_c = Ac^{-1} r_c
-// (with the partials of r_c . e_c), u += P e_c.
+// The two-level update's launches: the vector update with the restriction,
+// then the coarse rows with the prolongation.
 template <typename T, int ND, int NRP>
-std::function<int(const T *, T *, double *, const int *)> coarse_ops(hipStream_t s,
-                                                                     const tfm_mesh_t &m,
-                                                                     const tfm_coarse &c,
-                                                                     const uint8_t *con,
-                                                                     const T *inv) {
+void set_coarse_ops(Ops<T> &ops, hipStream_t s, const tfm_mesh_t &m, const tfm_coarse &c,
+                    const uint8_t *con, const T *inv) {
+  using Shape = CoarseShape<ND, NRP>;
   const CoarseView cv = c.view();
   const tfm_mesh_t mm = m;
-  return [=](const T *r, T *u, double *part, const int *flag) -> int {
-    hipLaunchKernelGGL((k_coarse_restrict<T, ND, NRP>), dim3((unsigned)cv.n_agg), dim3(BS), 0, s,
-                       mm, cv, con, r, flag);
+  const bool co = ops.scal;
+  const int chunks = Shape::chunks(m.n_nod, c.n_agg);
+  const unsigned grid = (unsigned)(c.n_agg * chunks);
+  const unsigned grid_c = Shape::AGGS > 1 ? (unsigned)((c.n_agg + Shape::AGGS - 1) / Shape::AGGS) : grid;
+  double *out = c.part + (size_t)grid * 2 * NRP;
+  ops.sets = out;
+  ops.n_sets = 1 + (int)(Shape::AGGS > 1 ? grid_c : (unsigned)c.n_agg);
+  ops.aux = c.aux;
+  ops.n_aux = (int)grid;
+  ops.update_coarse = [=](int it, T *x, T *r, T *u, const T *p, const T *sv, const T *minv,
+                          const PcgState &st, const double *pq, int n_pq) -> int {
+    const dim3 g(grid), t(Shape::THREADS);
+    if (it < 0)
+      hipLaunchKernelGGL((k_pcg_update_restrict<T, ND, NRP, false, true>), g, t, 0, s, mm, cv, con,
+                         chunks, 0, x, r, u, p, sv, minv, st, pq, n_pq);
+    else if (co)
+      hipLaunchKernelGGL((k_pcg_update_restrict<T, ND, NRP, true, false>), g, t, 0, s, mm, cv, con,
+                         chunks, it, x, r, u, p, sv, minv, st, pq, n_pq);
+    else
+      hipLaunchKernelGGL((k_pcg_update_restrict<T, ND, NRP, false, false>), g, t, 0, s, mm, cv,
+                         con, chunks, it, x, r, u, p, sv, minv, st, pq, n_pq);
     TFM_CHECK_LAUNCH();
-    hipLaunchKernelGGL((k_coarse_solve<T, NRP>), dim3((unsigned)((cv.n_c + 3) / 4)), dim3(BS), 0,
-                       s, cv, inv, flag);
-    TFM_CHECK_LAUNCH();
-    hipLaunchKernelGGL((k_coarse_prolong<T, ND, NRP>),
-                       dim3((unsigned)((mm.n_nod * NRP + 255) / 256)), dim3(256), 0, s, mm, cv, con,
-                       u, part, flag);
+    const int *flag = it < 0 ? cv.never : st.alldone;
+    constexpr bool SPLIT = Shape::AGGS == 1;  // chunks() may exceed 1
+    if (SPLIT && chunks == 4)
+      hipLaunchKernelGGL((k_coarse_apply<T, ND, NRP, SPLIT ? 4 : 1>), dim3(grid_c + 1), t, 0, s, mm,
+                         cv, con, inv, u, (int)grid, out, flag);
+    else if (SPLIT && chunks == 2)
+      hipLaunchKernelGGL((k_coarse_apply<T, ND, NRP, SPLIT ? 2 : 1>), dim3(grid_c + 1), t, 0, s, mm,
+                         cv, con, inv, u, (int)grid, out, flag);
+    else
+      hipLaunchKernelGGL((k_coarse_apply<T, ND, NRP, 1>), dim3(grid_c + 1), t, 0, s, mm, cv, con, inv,
+                         u, (int)grid, out, flag);
     TFM_CHECK_LAUNCH();
     return TFM_OK;
   };
@@ -1988,10 +2228,9 @@ int run_pcg(tfm_pcg *h, hipStream_t s, int64_t n_nod, Ops<T> &ops, const double 
   // whole multiples of the CU count, so that no CU runs a second round alone
   const unsigned gv = std::min<unsigned>(ops.scal ? std::max(RBV, RBW / NRP) : vcap,
                                          round_to_cus(grid_for(n_nod * NRP, BSV, RBW)));
-  // the coarse solve's partial sets follow the update's in part_upd
-  const int n_part = (int)gv + (ops.coarse ? 1 : 0);
-  double *const part_coarse = h->part_upd + (size_t)gv * 2 * NRP;
-  const int *never = h->coarse ? h->coarse->never : nullptr;
+  const bool two = (bool)ops.update_coarse;
+  const double *sets = two ? ops.sets : h->part_upd;
+  const int n_part = two ? ops.n_sets : (int)gv;
   std::vector<double> htol(NRP, -1.0), bnorm(NRP, 0.0), rprev(NRP, 0.0), rnow(NRP, 0.0);
   std::vector<int> fin(NRP, 1), stall(NRP, 0);
   for (int r = 0; r < nrhs; ++r) iters[r] = 0;
@@ -2034,15 +2273,18 @@ int run_pcg(tfm_pcg *h, hipStream_t s, int64_t n_nod, Ops<T> &ops, const double 
   auto seg_start_kernels = [&](int it, int mask, int cont, int running,
                                const SegInfo &seg) -> int {
     TFM_CHECK_HIP(hipMemcpyAsync(h->tol2, htol.data(), sizeof(double) * NRP, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL((k_pcg_seg_dots<T, ND, NRP>), dim3(gv), dim3(BS), 0, s, n_nod,
-                       (const T *)rv, uv, (const T *)pv, minv, st);
-    TFM_CHECK_LAUNCH();
-    if (ops.coarse) {
-      const int rc = ops.coarse(rv, uv, part_coarse, never);
+    if (two) {
+      const int rc = ops.update_coarse(-1, xv, rv, uv, pv, sv, minv, st, nullptr, 0);
       if (rc != TFM_OK) return rc;
+    } else {
+      hipLaunchKernelGGL((k_pcg_seg_dots<T, ND, NRP>), dim3(gv), dim3(BS), 0, s, n_nod,
+                         (const T *)rv, uv, (const T *)pv, minv, st);
+      TFM_CHECK_LAUNCH();
     }
     hipLaunchKernelGGL((k_pcg_seg_apply<T, ND, NRP>), dim3(gv), dim3(BS), 0, s, n_nod, it, mask,
-                       cont, running, seg, (const T *)uv, pv, sv, st, n_part, (int)gv);
+                       cont, running, seg, (const T *)uv, pv, sv, st, sets, n_part,
+                       two ? (const double *)ops.aux : (const double *)h->part_aux,
+                       two ? ops.n_aux : (int)gv);
     TFM_CHECK_LAUNCH();
     if (cont) return ops.spmv(pv, sv);
     return TFM_OK;
@@ -2083,32 +2325,32 @@ int run_pcg(tfm_pcg *h, hipStream_t s, int64_t n_nod, Ops<T> &ops, const double 
     for (; it < stop; ++it) {
       if (ops.scal) {
         hipLaunchKernelGGL((k_pcg_scal_dir<NRP>), dim3(1), dim3(BS), 0, s, it,
-                           (const double *)h->part_upd, n_part, st);
+                           sets, n_part, st);
         TFM_CHECK_LAUNCH();
       }
       const bool timed = h->timing && it % h->timing == 0;
       if (timed) TFM_CHECK_HIP(hipEventRecord(h->ev[2 * (it - start)], s));
       unsigned npq = 0;
-      int rc = ops.spmv_dir(uv, pv, sv, it, h->part_upd, n_part, st, &npq);
+      int rc = ops.spmv_dir(uv, pv, sv, it, sets, n_part, st, &npq);
       if (rc != TFM_OK) return rc;
       if (timed) TFM_CHECK_HIP(hipEventRecord(h->ev[2 * (it - start) + 1], s));
       if (ops.scal) {
         hipLaunchKernelGGL((k_pcg_scal_alpha<NRP>), dim3(1), dim3(1024), 0, s, it,
                            (const double *)h->part_pq, (int)npq, st);
         TFM_CHECK_LAUNCH();
+      }
+      if (two)
+        rc = ops.update_coarse(it, xv, rv, uv, pv, sv, minv, st, h->part_pq, (int)npq);
+      else if (ops.scal)
         hipLaunchKernelGGL((k_pcg_update<T, ND, NRP, true>), dim3(gv), dim3(BSV), 0, s, n_nod, it,
                            xv, rv, uv, (const T *)pv, (const T *)sv, minv, st,
                            (const double *)h->part_pq, (int)npq);
-      } else {
+      else
         hipLaunchKernelGGL((k_pcg_update<T, ND, NRP, false>), dim3(gv), dim3(BSV), 0, s, n_nod, it,
                            xv, rv, uv, (const T *)pv, (const T *)sv, minv, st,
                            (const double *)h->part_pq, (int)npq);
-      }
+      if (rc != TFM_OK) return rc;
       TFM_CHECK_LAUNCH();
-      if (ops.coarse) {
-        rc = ops.coarse(rv, uv, part_coarse, h->alldone);
-        if (rc != TFM_OK) return rc;
-      }
     }
     TFM_CHECK_HIP(hipMemcpyAsync(h->h_done, h->done, sizeof(int) * NRP, hipMemcpyDeviceToHost, s));
     TFM_CHECK_HIP(hipMemcpyAsync(h->h_scal, h->scal + (size_t)start * NRP * NSCAL,
@@ -2385,7 +2627,7 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
         return spmv_launch<double, ND, NRP>(s, m, sys->val64, xi, yo);
       };
       ops.residual = residual;
-      if (cs) ops.coarse = coarse_ops<double, ND, NRP>(s, m, *cs, sys->con, cs->inv64);
+      if (cs) set_coarse_ops<double, ND, NRP>(ops, s, m, *cs, sys->con, cs->inv64);
       return run_pcg<double, ND, NRP>(h, s, m.n_nod, ops, b, x, nrhs, rtol, inner_rtol,
                                       final_rtol, its, relres, out);
     };
@@ -2406,7 +2648,7 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
           return spmv_launch<float, ND, NRP>(s, m, sys->val32, xi, yo);
         };
         ops.residual = residual;
-        if (cs) ops.coarse = coarse_ops<float, ND, NRP>(s, m, *cs, sys->con, cs->inv32);
+        if (cs) set_coarse_ops<float, ND, NRP>(ops, s, m, *cs, sys->con, cs->inv32);
         rc = run_pcg<float, ND, NRP>(h, s, m.n_nod, ops, b, x, nrhs, rtol, inner_rtol, final_rtol,
                                      iters, relres, outer);
       }
