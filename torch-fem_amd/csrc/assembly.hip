@@ -659,118 +659,192 @@ __global__ void __launch_bounds__(64) k_assemble_nodes(tfm_mesh_t m, tfm_materia
   }
 }
 
-// =========================================================== element teams
-// Kernels below give each element a team of LG = next_pow2(NPE) lanes, one
-// lane per element node; Jacobians and gradients are summed across the team
-// with butterfly shuffles, so every lane ends with the full tensors.
-template <class E> constexpr int team_lanes() { return E::NPE <= 4 ? 4 : E::NPE <= 8 ? 8 : 32; }
+// ============================================================ point teams
+// Kernels below give each element one lane per Gauss point, 64 / NGP elements
+// to a wave (and a block). The nodal data and the shape-function derivatives
+// lie in LDS, so a lane forms the Jacobian and the nodal sums at its point by
+// itself: one lane per node instead needs a butterfly over the team for every
+// component of J and of grad u at every point, 864 LDS permutations per wave
+// of eight Hexa1 elements where this takes about 170 LDS reads.
+template <class E> constexpr int point_elems() { return 64 / E::NGP; }
+constexpr int odd(int n) { return n | 1; }  // row strides that spread over the LDS banks
 
-template <int LG, int NV> __device__ __forceinline__ void team_sum(double (&v)[NV]) {
-#pragma unroll
-  for (int off = 1; off < LG; off <<= 1)
-#pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] += __shfl_xor(v[i], off, LG);
-}
-
-// Per-lane geometry at Gauss point g: J^{-1}, detJ and this lane's column of B.
-template <class E, int LG>
-__device__ __forceinline__ double team_geometry(const double *Xj, bool act, int j, int g,
-                                                double (&Ji)[E::DIM][E::DIM], double *bj) {
-  constexpr int D = E::DIM;
+// dN/dxi of every point into LDS: tbl[g][k * NPE + N].
+template <class E>
+__device__ __forceinline__ void stage_table(double (&tbl)[E::NGP][odd(E::DIM * E::NPE)]) {
+  constexpr int R = E::DIM * E::NPE;
   const auto &T = shape_table<E>();
-  double Jv[D * D];
-  for (int i = 0; i < D; ++i)
-    for (int k = 0; k < D; ++k) Jv[i * D + k] = act ? T.dN[g][i][j] * Xj[k] : 0.0;
-  team_sum<LG, D * D>(Jv);
-  double J[D][D];
-  for (int i = 0; i < D; ++i)
-    for (int k = 0; k < D; ++k) J[i][k] = Jv[i * D + k];
-  const double det = inv_jac<D>(J, Ji);
-  for (int i = 0; i < D; ++i) {
-    double acc = 0.0;
-    if (act)
-      for (int k = 0; k < D; ++k) acc += Ji[i][k] * T.dN[g][k][j];
-    bj[i] = acc;
-  }
-  return det;
+  for (int q = threadIdx.x; q < E::NGP * R; q += blockDim.x) tbl[q / R][q % R] = (&T.dN[0][0][0])[q];
 }
 
-// Gradient H[a][i] = sum_N u[N][a] B[i][N], summed over the team (base.py:1052).
-template <int LG, int D, int NDOF>
-__device__ __forceinline__ void team_grad(const double *uj, const double *bj, double (&H)[NDOF * D]) {
-  for (int a = 0; a < NDOF; ++a)
-    for (int i = 0; i < D; ++i) H[a * D + i] = uj[a] * bj[i];
-  team_sum<LG, NDOF * D>(H);
+// Nodal values v[n][C] of the elements [e0, e0 + ne) into rows of LDS.
+template <class E, int C, int S>
+__device__ __forceinline__ void stage_nodal(const tfm_mesh_t &m, int64_t e0, int ne,
+                                            const double *v, double (*rows)[S]) {
+  for (int t = threadIdx.x; t < ne * E::NPE; t += blockDim.x) {
+    const int k = t / E::NPE, j = t - k * E::NPE;
+    const int64_t n = m.elements[e0 * E::NPE + t];
+    for (int c = 0; c < C; ++c) rows[k][j * C + c] = v[n * C + c];
+  }
 }
+
+// Sums over the nodes of v[N][a] dN_N/dxi_k at one point.
+template <class E, int C>
+__device__ __forceinline__ void point_sums(const double *row, const double *t,
+                                           double (&out)[C][E::DIM]) {
+  constexpr int NPE = E::NPE, D = E::DIM;
+  for (int a = 0; a < C; ++a)
+    for (int k = 0; k < D; ++k) out[a][k] = 0.0;
+#pragma unroll 4
+  for (int N = 0; N < NPE; ++N)
+    for (int a = 0; a < C; ++a)
+      for (int k = 0; k < D; ++k) out[a][k] += row[N * C + a] * t[k * NPE + N];
+}
+
+// J^{-1} and det J at one point.
+template <class E>
+__device__ __forceinline__ double point_geometry(const double *X, const double *t,
+                                                 double (&Ji)[E::DIM][E::DIM]) {
+  constexpr int D = E::DIM;
+  double S[D][D], J[D][D];
+  point_sums<E, D>(X, t, S);
+  for (int i = 0; i < D; ++i)
+    for (int k = 0; k < D; ++k) J[i][k] = S[k][i];
+  return inv_jac<D>(J, Ji);
+}
+
+// H[a][i] = sum_N u[N][a] B[i][N] at one point (base.py:1052).
+template <class E, int NDOF>
+__device__ __forceinline__ void point_grad(const double *u, const double *t,
+                                           const double (&Ji)[E::DIM][E::DIM],
+                                           double (&H)[NDOF * E::DIM]) {
+  constexpr int D = E::DIM;
+  double S[NDOF][D];
+  point_sums<E, NDOF>(u, t, S);
+  for (int a = 0; a < NDOF; ++a)
+    for (int i = 0; i < D; ++i) {
+      double acc = 0.0;
+      for (int k = 0; k < D; ++k) acc += Ji[i][k] * S[a][k];
+      H[a * D + i] = acc;
+    }
+}
+
+// Material parameters of a lane's element: the few of an isotropic or heat
+// layout in registers; the 81 (16) of a general stiffness in LDS where a team
+// shares them, and read in place where every lane has an element of its own
+// (64 of them would leave two waves per CU).
+template <class E, int MAT> struct PointParams {
+  static constexpr int NP = mat_nparam(MAT, E::DIM);
+  static constexpr bool REG = NP <= 9, LDS = !REG && E::NGP > 1;
+  static constexpr int ROWS = LDS ? point_elems<E>() : 1, STRIDE = LDS ? odd(NP) : 1;
+  double v[REG ? NP : 1];
+  const double *at;
+  __device__ __forceinline__ static void stage(const tfm_material_t &mat, int64_t e0, int ne,
+                                               double (&rows)[ROWS][STRIDE]) {
+    if constexpr (LDS)
+      for (int t = threadIdx.x; t < ne * NP; t += blockDim.x) rows[t / NP][t % NP] = mat.p0[e0 * NP + t];
+  }
+  __device__ __forceinline__ PointParams(const tfm_material_t &mat, int64_t e0, int el,
+                                         const double (&rows)[ROWS][STRIDE]) {
+    if constexpr (REG) {
+      for (int q = 0; q < NP; ++q) v[q] = mat_param<MAT, E::DIM>(mat, e0 + el, q);
+    } else {
+      at = LDS ? rows[LDS ? el : 0] : mat.p0 + (e0 + el) * NP;
+    }
+  }
+  __device__ __forceinline__ const double *get() const {
+    if constexpr (REG) return v;
+    else return at;
+  }
+};
 
 // Internal element forces fe[e][j][a] = sum_g w detJ s sum_i B[i][j] q[a][i]
 // with q = flux_prev + flux(grad u) (base.py:1050-1083 / 1250-1268); also
-// the Gauss-point means of grad u and q.
+// the Gauss-point means of grad u and q, and both per point. Lane (e, g) forms
+// q at its point and T[a][k] = w detJ s sum_i q[a][i] Jinv[i][k]; lane (e, j)
+// then adds T[a][k] dN_j/dxi_k over the points. Per-point values pass through
+// LDS, so that 64 lanes move the NQ * 64 / NGP consecutive values of a point.
+// Bound by the per-point arrays in memory where they are asked for, otherwise
+// by LDS reads. With one lane per node instead: Hexa1 43x37x40 with per-point
+// arrays (121 MB) 143 us, now 47; Hexa2 21x19x23 means only 87 us, now 14;
+// Tetra1 heat 63^3 98 us, now 58.
 template <class E, int NDOF, int MAT>
-__global__ void __launch_bounds__(256) k_internal_force(tfm_mesh_t m, tfm_material_t mat,
-                                                        const double *u, const double *qprev,
-                                                        double *fe, double *grad_mean,
-                                                        double *flux_mean, double *grad_gp,
-                                                        double *flux_gp) {
-  constexpr int NPE = E::NPE, NGP = E::NGP, D = E::DIM, NP = mat_nparam(MAT, D);
-  constexpr int LG = team_lanes<E>(), EPB = 256 / LG, NQ = NDOF * D;
-  __shared__ double MP[EPB][NP];
-  const int tid = threadIdx.x, slotE = tid / LG, j = tid % LG;
-  const int64_t blk = xcd_block();
-  const int64_t e = blk * EPB + slotE;
-  const bool live = e < m.n_elem;
-  const bool act = live && j < NPE;
-  for (int t = tid; t < EPB * NP; t += 256) {
-    const int k = t / NP, i = t - k * NP;
-    const int64_t ee = blk * EPB + k;
-    MP[k][i] = ee < m.n_elem ? mat_param<MAT, D>(mat, ee, i) : 0.0;
-  }
-  double Xj[D], uj[NDOF];
-  int64_t node = 0;
-  if (act) node = m.elements[e * NPE + j];
-  for (int d = 0; d < D; ++d) Xj[d] = act ? m.nodes[node * D + d] : 0.0;
-  for (int a = 0; a < NDOF; ++a) uj[a] = act ? u[node * NDOF + a] : 0.0;
+__global__ void __launch_bounds__(64) k_internal_force(tfm_mesh_t m, tfm_material_t mat,
+                                                       const double *u, const double *qprev,
+                                                       double *fe, double *grad_mean,
+                                                       double *flux_mean, double *grad_gp,
+                                                       double *flux_gp) {
+  constexpr int NPE = E::NPE, NGP = E::NGP, D = E::DIM;
+  constexpr int EPB = point_elems<E>(), NQ = NDOF * D, SQ = EPB * NQ;
+  __shared__ double tbl[NGP][odd(D * NPE)];
+  __shared__ double Xs[EPB][odd(NPE * D)], Us[EPB][odd(NPE * NDOF)];
+  using Params = PointParams<E, MAT>;
+  __shared__ double MP[Params::ROWS][Params::STRIDE];
+  __shared__ double st[64][odd(NQ)];  // per-point values of lane e * NGP + g
+  const int lane = threadIdx.x, el = lane / NGP, g = lane % NGP;
+  const int64_t e0 = xcd_block() * EPB;
+  const int ne = (int)(m.n_elem - e0 < EPB ? m.n_elem - e0 : EPB);
+  stage_table<E>(tbl);
+  stage_nodal<E, D>(m, e0, ne, m.nodes, Xs);
+  stage_nodal<E, NDOF>(m, e0, ne, u, Us);
+  Params::stage(mat, e0, ne, MP);
+  if (qprev)
+    for (int t = lane; t < NGP * SQ; t += 64) {
+      const int gg = t / SQ, r = t - gg * SQ, k = r / NQ;
+      if (k < ne) st[k * NGP + gg][r - k * NQ] = qprev[((int64_t)gg * m.n_elem + e0) * NQ + r];
+    }
   __syncthreads();
-  const double sc = live ? mat_scale(mat, e) : 0.0;
-  double fj[NDOF], Hs[NQ], Qs[NQ];
-  for (int a = 0; a < NDOF; ++a) fj[a] = 0.0;
-  for (int q = 0; q < NQ; ++q) Hs[q] = Qs[q] = 0.0;
-  for (int g = 0; g < NGP; ++g) {
-    double Ji[D][D], bj[D], H[NQ], Q[NQ];
-    const double det = team_geometry<E, LG>(Xj, act, j, g, Ji, bj);
-    team_grad<LG, D, NDOF>(uj, bj, H);
-    flux_from_grad<D, NDOF, MAT>(H, MP[slotE], Q);
-    if (qprev && live)
-      for (int q = 0; q < NQ; ++q) Q[q] += qprev[((int64_t)g * m.n_elem + e) * NQ + q];
-    const double wd = shape_table<E>().w[g] * det * sc;
-    for (int a = 0; a < NDOF; ++a) {
-      double acc = 0.0;
-      for (int i = 0; i < D; ++i) acc += bj[i] * Q[a * D + i];
-      fj[a] += wd * acc;
-    }
-    for (int q = 0; q < NQ; ++q) {
-      Hs[q] += H[q];
-      Qs[q] += Q[q];
-    }
-    if (live && (grad_gp || flux_gp)) {
-      const int64_t o = ((int64_t)g * m.n_elem + e) * NQ;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q)
-        if (q % LG == j) {  // component q is written by lane q % LG
-          if (grad_gp) grad_gp[o + q] = H[q];
-          if (flux_gp) flux_gp[o + q] = Q[q];
-        }
-    }
-  }
-  if (act)
-    for (int a = 0; a < NDOF; ++a) fe[(e * NPE + j) * NDOF + a] = fj[a];
-  if (live && (grad_mean || flux_mean)) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-      if (q % LG == j) {
-        if (grad_mean) grad_mean[e * NQ + q] = Hs[q] / NGP;
-        if (flux_mean) flux_mean[e * NQ + q] = Qs[q] / NGP;
+  double H[NQ], Q[NQ], T[NQ];
+  for (int q = 0; q < NQ; ++q) H[q] = Q[q] = T[q] = 0.0;
+  if (el < ne) {
+    double Ji[D][D];
+    const double det = point_geometry<E>(Xs[el], tbl[g], Ji);
+    point_grad<E, NDOF>(Us[el], tbl[g], Ji, H);
+    flux_from_grad<D, NDOF, MAT>(H, Params(mat, e0, el, MP).get(), Q);
+    if (qprev)
+      for (int q = 0; q < NQ; ++q) Q[q] += st[lane][q];
+    const double wd = shape_table<E>().w[g] * det * mat_scale(mat, e0 + el);
+    for (int a = 0; a < NDOF; ++a)
+      for (int k = 0; k < D; ++k) {
+        double acc = 0.0;
+        for (int i = 0; i < D; ++i) acc += Q[a * D + i] * Ji[i][k];
+        T[a * D + k] = wd * acc;
       }
+  }
+  // a per-point tensor and its mean over the points
+  auto emit = [&](const double (&v)[NQ], double *gp, double *mean) {
+    __syncthreads();
+    for (int q = 0; q < NQ; ++q) st[lane][q] = v[q];
+    __syncthreads();
+    if (gp)
+      for (int t = lane; t < NGP * SQ; t += 64) {
+        const int gg = t / SQ, r = t - gg * SQ, k = r / NQ;
+        if (k < ne) gp[((int64_t)gg * m.n_elem + e0) * NQ + r] = st[k * NGP + gg][r - k * NQ];
+      }
+    if (mean)
+      for (int t = lane; t < ne * NQ; t += 64) {
+        const int k = t / NQ, q = t - k * NQ;
+        double acc = 0.0;
+        for (int gg = 0; gg < NGP; ++gg) acc += st[k * NGP + gg][q];
+        mean[e0 * NQ + t] = acc / NGP;
+      }
+  };
+  if (grad_gp || grad_mean) emit(H, grad_gp, grad_mean);
+  if (flux_gp || flux_mean) emit(Q, flux_gp, flux_mean);
+  __syncthreads();
+  for (int q = 0; q < NQ; ++q) st[lane][q] = T[q];
+  __syncthreads();
+  for (int t = lane; t < ne * NPE; t += 64) {
+    const int k = t / NPE, j = t - k * NPE;
+    double f[NDOF];
+    for (int a = 0; a < NDOF; ++a) f[a] = 0.0;
+#pragma unroll 4
+    for (int gg = 0; gg < NGP; ++gg)
+      for (int kk = 0; kk < D; ++kk) {
+        const double b = tbl[gg][kk * NPE + j];
+        for (int a = 0; a < NDOF; ++a) f[a] += st[k * NGP + gg][a * D + kk] * b;
+      }
+    for (int a = 0; a < NDOF; ++a) fe[(e0 * NPE + t) * NDOF + a] = f[a];
   }
 }
 
@@ -873,53 +947,57 @@ __global__ void __launch_bounds__(64) k_assemble_elements(tfm_mesh_t m, const do
   }
 }
 
-// Sensitivities of lam^T K(p) u per element (see tfm_sensitivity in tfm.h).
+// Sensitivities of lam^T K(p) u per element (see tfm_sensitivity in tfm.h):
+// a lane per Gauss point, whose geometry serves every right-hand side.
+// Hexa2 21x19x23 with 12 right-hand sides: 1385 us with a lane per node and
+// the geometry formed for each, now 80; Hexa1 47x41x52 with one 186 us, now 28.
 template <class E, int NDOF, int MAT>
-__global__ void __launch_bounds__(256) k_sensitivity(tfm_mesh_t m, tfm_material_t mat,
-                                                     const double *u, const double *lam,
-                                                     int nrhs, double sign, double *out) {
+__global__ void __launch_bounds__(64) k_sensitivity(tfm_mesh_t m, tfm_material_t mat,
+                                                    const double *u, const double *lam,
+                                                    int nrhs, double sign, double *out) {
   constexpr int NPE = E::NPE, NGP = E::NGP, D = E::DIM, NP = mat_nparam(MAT, D);
-  constexpr int LG = team_lanes<E>(), EPB = 256 / LG, NQ = NDOF * D;
+  constexpr int EPB = point_elems<E>(), NQ = NDOF * D;
   constexpr bool ISO = (MAT == TFM_MAT_ISO || MAT == TFM_MAT_HEAT_ISO);
-  constexpr int NO = (MAT == TFM_MAT_ISO ? 2 : MAT == TFM_MAT_HEAT_ISO ? 1 : NP) + 1;
-  constexpr int PER = (NO - 1 + LG - 1) / LG;  // general layouts: outputs per lane
-  __shared__ double MP[EPB][NP];
-  const int tid = threadIdx.x, slotE = tid / LG, j = tid % LG;
-  const int64_t blk = xcd_block();
-  const int64_t e = blk * EPB + slotE;
-  const bool live = e < m.n_elem;
-  const bool act = live && j < NPE;
-  for (int t = tid; t < EPB * NP; t += 256) {
-    const int k = t / NP, i = t - k * NP;
-    const int64_t ee = blk * EPB + k;
-    MP[k][i] = ee < m.n_elem ? mat_param<MAT, D>(mat, ee, i) : 0.0;
-  }
-  double Xj[D];
-  int64_t node = 0;
-  if (act) node = m.elements[e * NPE + j];
-  for (int d = 0; d < D; ++d) Xj[d] = act ? m.nodes[node * D + d] : 0.0;
+  constexpr int NI = MAT == TFM_MAT_ISO ? 2 : 1, NO = (ISO ? NI : NP) + 1;
+  __shared__ double tbl[NGP][odd(D * NPE)];
+  __shared__ double Xs[EPB][odd(NPE * D)];
+  __shared__ double Us[EPB][odd(NPE * NDOF)], Ls[EPB][odd(NPE * NDOF)];
+  using Params = PointParams<E, MAT>;
+  __shared__ double MP[Params::ROWS][Params::STRIDE];
+  // general layouts: w detJ s grad(lam), sym(grad u) or grad u, and the energy
+  __shared__ double st[ISO ? 1 : 64][odd(2 * NQ + 1)];
+  const int lane = threadIdx.x, el = lane / NGP, g = lane % NGP;
+  const int64_t e0 = xcd_block() * EPB;
+  const int ne = (int)(m.n_elem - e0 < EPB ? m.n_elem - e0 : EPB);
+  const bool live = el < ne;
+  stage_table<E>(tbl);
+  stage_nodal<E, D>(m, e0, ne, m.nodes, Xs);
+  Params::stage(mat, e0, ne, MP);
   __syncthreads();
-  const double sc = live ? mat_scale(mat, e) : 0.0;
+  const double sc = live ? mat_scale(mat, e0 + el) : 0.0;
+  const Params mp(mat, e0, live ? el : 0, MP);
+  double Ji[D][D], wd = 0.0;
+  for (int i = 0; i < D; ++i)
+    for (int k = 0; k < D; ++k) Ji[i][k] = 0.0;
+  if (live) wd = shape_table<E>().w[g] * point_geometry<E>(Xs[el], tbl[g], Ji);
   const int64_t ndofs = m.n_nod * NDOF;
   for (int r = 0; r < nrhs; ++r) {
-    double uj[NDOF], lj[NDOF];
-    for (int a = 0; a < NDOF; ++a) {
-      uj[a] = act ? u[r * ndofs + node * NDOF + a] : 0.0;
-      lj[a] = act ? lam[r * ndofs + node * NDOF + a] : 0.0;
-    }
-    double iso_acc[2] = {0.0, 0.0}, gen_acc[PER > 0 ? PER : 1], sacc = 0.0;
-    for (int o = 0; o < (PER > 0 ? PER : 1); ++o) gen_acc[o] = 0.0;
-    for (int g = 0; g < NGP; ++g) {
-      double Ji[D][D], bj[D], Hu[NQ], Hl[NQ], Q[NQ];
-      const double det = team_geometry<E, LG>(Xj, act, j, g, Ji, bj);
-      team_grad<LG, D, NDOF>(uj, bj, Hu);
-      team_grad<LG, D, NDOF>(lj, bj, Hl);
-      const double wd = shape_table<E>().w[g] * det;
+    __syncthreads();
+    stage_nodal<E, NDOF>(m, e0, ne, u + r * ndofs, Us);
+    stage_nodal<E, NDOF>(m, e0, ne, lam + r * ndofs, Ls);
+    __syncthreads();
+    double *o = out + ((int64_t)r * m.n_elem + e0) * NO;
+    double acc[3] = {0.0, 0.0, 0.0};
+    double Hu[NQ], Hl[NQ];
+    if (live) {
+      double Q[NQ];
+      point_grad<E, NDOF>(Us[el], tbl[g], Ji, Hu);
+      point_grad<E, NDOF>(Ls[el], tbl[g], Ji, Hl);
       // d/dscale: sum_g w detJ Hl : flux(Hu)
-      flux_from_grad<D, NDOF, MAT>(Hu, MP[slotE], Q);
+      flux_from_grad<D, NDOF, MAT>(Hu, mp.get(), Q);
       double en = 0.0;
       for (int q = 0; q < NQ; ++q) en += Hl[q] * Q[q];
-      sacc += wd * en;
+      acc[2] = wd * en;
       if constexpr (MAT == TFM_MAT_ISO) {
         double tl = 0.0, tu = 0.0, dd = 0.0;
         for (int i = 0; i < D; ++i) {
@@ -928,46 +1006,47 @@ __global__ void __launch_bounds__(256) k_sensitivity(tfm_mesh_t m, tfm_material_
         }
         for (int i = 0; i < D; ++i)
           for (int k = 0; k < D; ++k) dd += Hl[i * D + k] * (Hu[i * D + k] + Hu[k * D + i]);
-        iso_acc[0] += wd * sc * tl * tu;
-        iso_acc[1] += wd * sc * dd;
+        acc[0] = wd * sc * tl * tu;
+        acc[1] = wd * sc * dd;
       } else if constexpr (MAT == TFM_MAT_HEAT_ISO) {
         double dd = 0.0;
         for (int i = 0; i < D; ++i) dd += Hl[i] * Hu[i];
-        iso_acc[0] += wd * sc * dd;
-      } else {
-        // general: d/dC[i,J,k,L] = Hl[i][J] eps_u[k][L]; heat: d/dKAPPA[i,j] =
-        // dT_l/dx_i dT_u/dx_j. Output c lives on lane c % LG, slot c / LG;
-        // the loops are unrolled so no register array is indexed at run time.
-        // mechanics pairs Hl with the strain sym(Hu): the residual depends on
-        // C only through C : sym(grad u) (elasticity.py:121-123)
-        double Hv[NQ];
-        for (int x = 0; x < NQ; ++x) Hv[x] = Hu[x];
-        if constexpr (MAT == TFM_MAT_GENERAL)
-          for (int k = 0; k < D; ++k)
-            for (int l = 0; l < D; ++l) Hv[k * D + l] = 0.5 * (Hu[k * D + l] + Hu[l * D + k]);
-#pragma unroll
-        for (int x = 0; x < NQ; ++x)
-#pragma unroll
-          for (int y = 0; y < NQ; ++y) {
-            const int c = x * NQ + y;
-            if (c % LG == j) gen_acc[c / LG] += wd * sc * Hl[x] * Hv[y];
-          }
+        acc[0] = wd * sc * dd;
       }
     }
-    if (!live) continue;
-    double *o = out + ((int64_t)r * m.n_elem + e) * NO;
     if constexpr (ISO) {
-      if (j == 0) {
-        o[0] = sign * iso_acc[0];
-        if (MAT == TFM_MAT_ISO) o[1] = sign * iso_acc[1];
-        o[NO - 1] = sign * sacc;
+#pragma unroll
+      for (int off = 1; off < NGP; off <<= 1)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) acc[c] += __shfl_xor(acc[c], off, 64);
+      if (live && g == 0) {
+        for (int c = 0; c < NI; ++c) o[el * NO + c] = sign * acc[c];
+        o[el * NO + NI] = sign * acc[2];
       }
     } else {
-      for (int q = 0; q < PER; ++q) {
-        const int c = j + q * LG;
-        if (c < NP) o[c] = sign * gen_acc[q];
+      // general: d/dC[i,J,k,L] = Hl[i][J] eps_u[k][L]; heat: d/dKAPPA[i,j] =
+      // dT_l/dx_i dT_u/dx_j. Mechanics pairs Hl with the strain sym(Hu): the
+      // residual depends on C only through C : sym(grad u)
+      // (elasticity.py:121-123)
+      if (live) {
+        for (int x = 0; x < NQ; ++x) {
+          st[lane][x] = wd * sc * Hl[x];
+          double h = Hu[x];
+          if constexpr (MAT == TFM_MAT_GENERAL) h = 0.5 * (Hu[x] + Hu[(x % D) * D + x / D]);
+          st[lane][NQ + x] = h;
+        }
+        st[lane][2 * NQ] = acc[2];
       }
-      if (j == 0) o[NO - 1] = sign * sacc;
+      __syncthreads();
+      for (int t = lane; t < ne * NO; t += 64) {
+        const int k = t / NO, c = t - k * NO;
+        double v = 0.0;
+        for (int gg = 0; gg < NGP; ++gg) {
+          const double *S = st[k * NGP + gg];
+          v += c < NP ? S[c / NQ] * S[NQ + c % NQ] : S[2 * NQ];
+        }
+        o[t] = sign * v;
+      }
     }
   }
 }
@@ -1063,10 +1142,10 @@ int launch_internal_force(hipStream_t s, const tfm_mesh_t &m, const tfm_material
                           double *grad_mean, double *flux_mean, double *grad_gp,
                           double *flux_gp, double *work) {
   TFM_DISPATCH_ALL(m, mat, {
-    constexpr int EPB = 256 / team_lanes<ET>();
+    constexpr int EPB = point_elems<ET>();
     if (m.n_elem > 0) {
       const unsigned nb = (unsigned)((m.n_elem + EPB - 1) / EPB);
-      hipLaunchKernelGGL((k_internal_force<ET, ND, MK>), dim3(nb), dim3(256), 0, s, m, mat, u,
+      hipLaunchKernelGGL((k_internal_force<ET, ND, MK>), dim3(nb), dim3(64), 0, s, m, mat, u,
                          flux_prev, work, grad_mean, flux_mean, grad_gp, flux_gp);
       TFM_CHECK_LAUNCH();
     }
@@ -1126,9 +1205,9 @@ int launch_sensitivity(hipStream_t s, const tfm_mesh_t &m, const tfm_material_t 
                        const double *u, const double *lam, int nrhs, double sign, double *out) {
   if (m.n_elem == 0 || nrhs == 0) return TFM_OK;
   TFM_DISPATCH_ALL(m, mat, {
-    constexpr int EPB = 256 / team_lanes<ET>();
+    constexpr int EPB = point_elems<ET>();
     const unsigned nb = (unsigned)((m.n_elem + EPB - 1) / EPB);
-    hipLaunchKernelGGL((k_sensitivity<ET, ND, MK>), dim3(nb), dim3(256), 0, s, m, mat, u, lam,
+    hipLaunchKernelGGL((k_sensitivity<ET, ND, MK>), dim3(nb), dim3(64), 0, s, m, mat, u, lam,
                        nrhs, sign, out);
     TFM_CHECK_LAUNCH();
   });
