@@ -98,3 +98,11 @@ def test_forces_fluxes_and_sensitivities(name, n, general):
         ref = -torch.einsum("ei,eij,ej->e", lam[r][idx], k0.reshape(n, idx.shape[1], -1), u[r][idx])
         assert close(out[r, :, -1], ref)
         assert close((out[r, :, :-1] * pars).sum(1), ref)
+
+
+@pytest.mark.parametrize("name,n,general", SIZES)
+def test_element_matrices(name, n, general):
+    """Element counts around the elements of a block (16, 4, 1)."""
+    m, o = model(name, n, general)
+    k0 = o.integrate(torch.zeros(o.n_dofs, dtype=DT), need_k=True)[0]
+    assert close(m.k0().reshape(k0.shape), k0)
