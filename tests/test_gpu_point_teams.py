@@ -106,3 +106,26 @@ def test_element_matrices(name, n, general):
     m, o = model(name, n, general)
     k0 = o.integrate(torch.zeros(o.n_dofs, dtype=DT), need_k=True)[0]
     assert close(m.k0().reshape(k0.shape), k0)
+
+
+@pytest.mark.parametrize("orphans", [False, True])
+@pytest.mark.parametrize("name,n,general", SIZES)
+def test_assembly_of_element_matrices(name, n, general, orphans):
+    """Any (unsymmetric) element matrices; nodes of no element first and last.
+    At most 24 terms per entry: 24 eps = 2.7e-15 of the largest sum."""
+    m, o = model(name, n, general)
+    if orphans:
+        X, el = m.nodes, m.elements
+        X = torch.cat([X[:1], X[:1], X, X[:2]])
+        m = type(m)(X, el + 2, None)
+    g = torch.Generator().manual_seed(3)
+    W = m._pattern.npe * m.n_dof_per_node
+    k = torch.randn(n, W, W, generator=g, dtype=DT)
+    con = torch.nonzero(torch.rand(m.n_dofs, generator=g) < 0.2).reshape(-1)
+    K = m.assemble_matrix(k.cuda(), con.cuda()).to_dense().cpu()
+    idx = m.idx.cpu().long()
+    ref = torch.zeros(m.n_dofs, m.n_dofs, dtype=DT)
+    ref.index_put_((idx[:, :, None].expand_as(k), idx[:, None, :].expand_as(k)), k, accumulate=True)
+    ref[con], ref[:, con] = 0.0, 0.0
+    ref[con, con] = 1.0
+    assert float((K - ref).abs().max()) <= 3e-15 * float(ref.abs().max()) * 24

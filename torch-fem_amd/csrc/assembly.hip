@@ -3,6 +3,8 @@
 // copy for the mixed-precision solver is rounded from the FP64 sums.
 #include "tfm_common.h"
 
+#include <type_traits>
+
 namespace tfm {
 
 // Shape-function tables, evaluated at compile time (see tfm_common.h).
@@ -436,6 +438,100 @@ __global__ void __launch_bounds__(64) k_assemble_rows(tfm_mesh_t m, tfm_material
   }
 }
 
+// What the rows of a tile of NW nodes need: first values, adjacency, the slot
+// of the node itself and the Dirichlet bits of its DOFs.
+template <int NW> struct Tile {
+  int64_t vb[NW + 1];
+  int a0[NW], deg[NW], self[NW], crow[NW];
+};
+
+template <int NDOF, int NW>
+__device__ __forceinline__ void tile_load(const tfm_mesh_t &m, int64_t n0, const uint8_t *con,
+                                          Tile<NW> &tile) {
+  const int lane = threadIdx.x;
+  if (lane < NW) {
+    const int64_t nn = n0 + lane;
+    const bool ok = nn < m.n_nod;
+    tile.a0[lane] = ok ? m.adj_ptr[nn] : 0;
+    tile.deg[lane] = ok ? m.adj_ptr[nn + 1] - m.adj_ptr[nn] : 0;
+    tile.vb[lane] = m.val_ptr[ok ? nn : m.n_nod];
+    tile.self[lane] = -1;
+    int cr = 0;
+    for (int a = 0; a < NDOF; ++a) cr |= ok && con[nn * NDOF + a] ? 1 << a : 0;
+    tile.crow[lane] = cr;
+    if (lane == NW - 1) tile.vb[NW] = m.val_ptr[nn + 1 < m.n_nod ? nn + 1 : m.n_nod];
+  }
+}
+
+// The tile's accumulated rows, with the Dirichlet rows and columns replaced by
+// the identity, to the value arrays.
+template <int NDOF, int NW>
+__device__ __forceinline__ void tile_epilogue(const tfm_mesh_t &m, int64_t n0, double *acc,
+                                              int stride, const unsigned char *cmask,
+                                              const Tile<NW> &tile, double *v64, float *v32,
+                                              double *dblk, int diff32) {
+  constexpr int ND2 = NDOF * NDOF;
+  const int lane = threadIdx.x;
+  // the tile's rows are contiguous in the value arrays: [tile.vb[0], tile.vb[NW])
+  const int64_t vb0 = tile.vb[0];
+  const int total = (int)(tile.vb[NW] - vb0);
+  int wq = 0, beg = 0, end = (int)(tile.vb[1] - vb0);  // lane's node and its value range
+  for (int q = lane; q < total; q += 64) {
+    while (end <= q) {
+      ++wq;
+      beg = end;
+      end = (int)(tile.vb[wq + 1] - vb0);
+    }
+    const int64_t nn = n0 + wq;
+    const int deg = tile.deg[wq];
+    const int ql = q - beg;
+    if (deg == 0) {  // orphan node: only its diagonal is stored (base.py:89-90)
+      const double v = (tile.crow[wq] >> ql) & 1 ? 1.0 : 0.0;
+      if (v64) v64[vb0 + q] = v;
+      if (v32) v32[vb0 + q] = (float)v;
+      continue;
+    }
+    const int L = NDOF * deg;
+    int a = 0, rem = ql;  // ql = a L + rem
+    for (int k = 1; k < NDOF; ++k)
+      if (rem >= L) {
+        rem -= L;
+        ++a;
+      }
+    const int p = rem / NDOF, b = rem - p * NDOF;
+    const int self = tile.self[wq];
+    double *A = acc + wq * stride;
+    double v = A[ql];
+    if (((tile.crow[wq] >> a) & 1) || ((cmask[wq * m.max_deg + p] >> b) & 1))
+      v = (p == self && a == b) ? 1.0 : 0.0;  // row == col
+    A[ql] = v;
+    if (v64) v64[vb0 + q] = v;
+    if (v32 && (p != self || !diff32)) v32[vb0 + q] = (float)v;
+    if (p == self) dblk[nn * ND2 + a * NDOF + b] = v;
+  }
+  for (int q = lane; q < NW * ND2; q += 64) {  // orphan diagonal blocks
+    const int ww = q / ND2, ab = q - ww * ND2, a = ab / NDOF, b = ab - a * NDOF;
+    const int64_t nn = n0 + ww;
+    if (nn < m.n_nod && tile.deg[ww] == 0)
+      dblk[nn * ND2 + ab] = (a == b && ((tile.crow[ww] >> a) & 1)) ? 1.0 : 0.0;
+  }
+  // FP32 difference form: the diagonal block holds the row sums of the
+  // final FP64 values, added in ascending slot order
+  if (v32 && diff32) {
+    __syncthreads();
+    for (int q = lane; q < NW * ND2; q += 64) {
+      const int ww = q / ND2, ab = q - ww * ND2, a = ab / NDOF, b = ab - a * NDOF;
+      const int deg = tile.deg[ww];
+      if (n0 + ww >= m.n_nod || deg == 0) continue;
+      const int L = NDOF * deg;
+      const double *A = acc + ww * stride;
+      double r = 0.0;
+      for (int p = 0; p < deg; ++p) r += A[a * L + p * NDOF + b];
+      v32[tile.vb[ww] + a * L + tile.self[ww] * NDOF + b] = (float)r;
+    }
+  }
+}
+
 // Node-tiled assembly. A 64-lane block assembles the rows of NW consecutive
 // nodes. A node owns NPE * IP lanes: IP of its incident elements are taken at
 // once (incidence t = r IP + ip in round r), each by NPE lanes, lane j for the
@@ -485,8 +581,7 @@ __global__ void __launch_bounds__(64) k_assemble_nodes(tfm_mesh_t m, tfm_materia
   __shared__ double tw[NGP];
   __shared__ double Xs[NG][XS];   // [group][N * D + c]
   __shared__ double Gm[NG][GS];   // [group][g * GW + ...]
-  __shared__ int64_t s_vb[NW + 1];
-  __shared__ int s_a0[NW], s_deg[NW], s_self[NW], s_crow[NW];
+  __shared__ Tile<NW> tile;
 
   const int lane = threadIdx.x;
   const int w = lane / LPN, ip = (lane / NPE) % IP, j = lane % NPE, grp = w * IP + ip;
@@ -500,18 +595,7 @@ __global__ void __launch_bounds__(64) k_assemble_nodes(tfm_mesh_t m, tfm_materia
     inc0 = m.ne_ptr[n];
     ninc = m.ne_ptr[n + 1] - inc0;
   }
-  if (lane < NW) {
-    const int64_t nn = n0 + lane;
-    const bool ok = nn < m.n_nod;
-    s_a0[lane] = ok ? m.adj_ptr[nn] : 0;
-    s_deg[lane] = ok ? m.adj_ptr[nn + 1] - m.adj_ptr[nn] : 0;
-    s_vb[lane] = m.val_ptr[ok ? nn : m.n_nod];
-    s_self[lane] = -1;
-    int cr = 0;
-    for (int a = 0; a < NDOF; ++a) cr |= ok && con[nn * NDOF + a] ? 1 << a : 0;
-    s_crow[lane] = cr;
-    if (lane == NW - 1) s_vb[NW] = m.val_ptr[nn + 1 < m.n_nod ? nn + 1 : m.n_nod];
-  }
+  tile_load<NDOF, NW>(m, n0, con, tile);
   const auto &T = shape_table<E>();
   for (int q = lane; q < NGP * D * NPE; q += 64) tbl[q / (D * NPE)][q % (D * NPE)] = (&T.dN[0][0][0])[q];
   for (int q = lane; q < NGP; q += 64) tw[q] = T.w[q];
@@ -529,7 +613,7 @@ __global__ void __launch_bounds__(64) k_assemble_nodes(tfm_mesh_t m, tfm_materia
       nbr[c] = -1;
       if (q < nq) {
         const int ww = q / m.max_deg, p = q - ww * m.max_deg;
-        if (p < s_deg[ww]) nbr[c] = m.adj[s_a0[ww] + p];
+        if (p < tile.deg[ww]) nbr[c] = m.adj[tile.a0[ww] + p];
       }
     }
   };
@@ -591,7 +675,7 @@ __global__ void __launch_bounds__(64) k_assemble_nodes(tfm_mesh_t m, tfm_materia
       const int i = il[b];
       if (act) {
         for (int d = 0; d < D; ++d) Xs[grp][j * D + d] = X[b][d];
-        if (r0 + b == 0 && ip == 0 && j == i) s_self[w] = P[b];
+        if (r0 + b == 0 && ip == 0 && j == i) tile.self[w] = P[b];
       }
       __syncthreads();
       if (act && j < NGP) {  // lane g = j: the geometry of point g
@@ -655,7 +739,7 @@ __global__ void __launch_bounds__(64) k_assemble_nodes(tfm_mesh_t m, tfm_materia
       for (int st = 0; st < IP; ++st) {
         if (act && ip == st) {
           double *A = acc + w * stride;
-          const int L = NDOF * s_deg[w];
+          const int L = NDOF * tile.deg[w];
           for (int a = 0; a < NDOF; ++a)
             for (int c = 0; c < NDOF; ++c) A[a * L + P[b] * NDOF + c] += blk[a * NDOF + c];
         }
@@ -669,64 +753,7 @@ __global__ void __launch_bounds__(64) k_assemble_nodes(tfm_mesh_t m, tfm_materia
     cm_con(q0, nbr);
   }
   __syncthreads();
-  // the tile's rows are contiguous in the value arrays: [s_vb[0], s_vb[NW])
-  const int64_t vb0 = s_vb[0];
-  const int total = (int)(s_vb[NW] - vb0);
-  int wq = 0, beg = 0, end = (int)(s_vb[1] - vb0);  // lane's node and its value range
-  for (int q = lane; q < total; q += 64) {
-    while (end <= q) {
-      ++wq;
-      beg = end;
-      end = (int)(s_vb[wq + 1] - vb0);
-    }
-    const int64_t nn = n0 + wq;
-    const int deg = s_deg[wq];
-    const int ql = q - beg;
-    if (deg == 0) {  // orphan node: only its diagonal is stored (base.py:89-90)
-      const double v = (s_crow[wq] >> ql) & 1 ? 1.0 : 0.0;
-      if (v64) v64[vb0 + q] = v;
-      if (v32) v32[vb0 + q] = (float)v;
-      continue;
-    }
-    const int L = NDOF * deg;
-    int a = 0, rem = ql;  // ql = a L + rem
-    for (int k = 1; k < NDOF; ++k)
-      if (rem >= L) {
-        rem -= L;
-        ++a;
-      }
-    const int p = rem / NDOF, b = rem - p * NDOF;
-    const int self = s_self[wq];
-    double *A = acc + wq * stride;
-    double v = A[ql];
-    if (((s_crow[wq] >> a) & 1) || ((cmask[wq * m.max_deg + p] >> b) & 1))
-      v = (p == self && a == b) ? 1.0 : 0.0;  // row == col
-    A[ql] = v;
-    if (v64) v64[vb0 + q] = v;
-    if (v32 && (p != self || !diff32)) v32[vb0 + q] = (float)v;
-    if (p == self) dblk[nn * ND2 + a * NDOF + b] = v;
-  }
-  for (int q = lane; q < NW * ND2; q += 64) {  // orphan diagonal blocks
-    const int ww = q / ND2, ab = q - ww * ND2, a = ab / NDOF, b = ab - a * NDOF;
-    const int64_t nn = n0 + ww;
-    if (nn < m.n_nod && s_deg[ww] == 0)
-      dblk[nn * ND2 + ab] = (a == b && ((s_crow[ww] >> a) & 1)) ? 1.0 : 0.0;
-  }
-  // FP32 difference form: the diagonal block holds the row sums of the
-  // final FP64 values, added in ascending slot order
-  if (v32 && diff32) {
-    __syncthreads();
-    for (int q = lane; q < NW * ND2; q += 64) {
-      const int ww = q / ND2, ab = q - ww * ND2, a = ab / NDOF, b = ab - a * NDOF;
-      const int deg = s_deg[ww];
-      if (n0 + ww >= m.n_nod || deg == 0) continue;
-      const int L = NDOF * deg;
-      const double *A = acc + ww * stride;
-      double r = 0.0;
-      for (int p = 0; p < deg; ++p) r += A[a * L + p * NDOF + b];
-      v32[s_vb[ww] + a * L + s_self[ww] * NDOF + b] = (float)r;
-    }
-  }
+  tile_epilogue<NDOF, NW>(m, n0, acc, stride, cmask, tile, v64, v32, dblk, diff32);
 }
 
 // ============================================================ point teams
@@ -945,75 +972,96 @@ __global__ void k_gather_nodes(tfm_mesh_t m, const double *fe, double *F) {
   F[t] = acc;
 }
 
-// Assembly from given element matrices kin [E, W, W]: same node-row order and
-// Dirichlet epilogue as k_assemble_rows.
-template <int NDOF>
+// Assembly from given element matrices kin [E, W, W]: LPN lanes per node, NW =
+// 64 / LPN consecutive nodes per block. The NDOF rows that an element gives a
+// node are NDOF * W consecutive values of kin; the lanes load those of U
+// elements together and add them into the node's rows in LDS one element after
+// the other (ascending, a fixed order, one writer per entry), so every value of
+// kin is read once, in whole lines. The tile leaves as in k_assemble_nodes.
+// Bound by reading kin: Hexa1 43x37x40 135 us (420 MB in and out, 3.1 TB/s), 297
+// us with a gather of every entry from its elements; Hexa2 13x15x11 35 us (99).
+// Two or eight elements at once took 135 and 148 us.
+// lanes per node: the fewest that hold its values of an element in three rounds
+// (72 of Hexa1: 32 lanes and 135 us on 43x37x40; 64 lanes with two rounds, of
+// which the second is nearly empty, 145 us)
+constexpr int assemble_lanes(int npe, int nd) {
+  int l = 4;
+  while (l < 64 && l * 3 < npe * nd * nd) l *= 2;
+  return l;
+}
+
+template <int NPE, int NDOF>
 __global__ void __launch_bounds__(64) k_assemble_elements(tfm_mesh_t m, const double *kin,
                                                           const uint8_t *con, double *v64,
                                                           float *v32, double *dblk, int diff32) {
-  constexpr int ND2 = NDOF * NDOF;
-  extern __shared__ signed char slot_dyn[];  // [max_inc * max_deg]
-  const int64_t n = xcd_block();
-  const int tid = threadIdx.x;
-  const int npe = m.npe, W = npe * NDOF;
-  const int a0 = m.adj_ptr[n];
-  const int deg = m.adj_ptr[n + 1] - a0;
-  const int64_t vb = m.val_ptr[n];
-  if (deg == 0) {
-    if (tid < NDOF) {
-      const double v = con[n * NDOF + tid] ? 1.0 : 0.0;
-      if (v64) v64[vb + tid] = v;
-      if (v32) v32[vb + tid] = (float)v;
-    }
-    for (int t = tid; t < ND2; t += 64) {
-      const int a = t / NDOF, b = t - a * NDOF;
-      dblk[n * ND2 + t] = (a == b && con[n * NDOF + a]) ? 1.0 : 0.0;
-    }
-    return;
+  constexpr int W = NPE * NDOF, ND2 = NDOF * NDOF, NV = NDOF * W;
+  constexpr int LPN = assemble_lanes(NPE, NDOF), NW = 64 / LPN;
+  constexpr int IR = (NV + LPN - 1) / LPN, U = 4;  // values per lane and element, elements
+  extern __shared__ double acc[];  // rows [NW][ND2 * max_deg], Dirichlet bits [NW][max_deg]
+  __shared__ Tile<NW> tile;
+  const int lane = threadIdx.x, w = lane / LPN, l = lane % LPN;
+  const int64_t n0 = xcd_block() * (int64_t)NW;
+  const int64_t n = n0 + w;
+  const int stride = ND2 * m.max_deg;
+  unsigned char *cmask = reinterpret_cast<unsigned char *>(acc + NW * stride);
+  int inc0 = 0, ninc = 0;
+  if (n < m.n_nod) {
+    inc0 = m.ne_ptr[n];
+    ninc = m.ne_ptr[n + 1] - inc0;
+    if (ninc == 0) inc0 = 0;  // an index that can be read
   }
-  const int inc0 = m.ne_ptr[n], ninc = m.ne_ptr[n + 1] - inc0;
-  for (int t = tid; t < ninc * deg; t += 64) slot_dyn[t] = -1;
+  int most = ninc;  // over the tile
+#pragma unroll
+  for (int off = LPN; off < 64; off <<= 1) most = max(most, __shfl_xor(most, off, 64));
+  tile_load<NDOF, NW>(m, n0, con, tile);
+  for (int q = lane; q < NW * stride; q += 64) acc[q] = 0.0;
   __syncthreads();
-  for (int t = tid; t < ninc * npe; t += 64) {
-    const int k = t / npe, j = t - k * npe;
-    const int64_t e = m.ne_elem[inc0 + k];
-    slot_dyn[k * deg + m.epos[(e * npe + m.ne_loc[inc0 + k]) * npe + j]] = (signed char)j;
+  const int deg = tile.deg[w], L = NDOF * deg;
+  for (int p = l; p < deg; p += LPN) {
+    const int64_t c = m.adj[tile.a0[w] + p];
+    int bits = 0;
+    for (int b = 0; b < NDOF; ++b) bits |= con[c * NDOF + b] ? 1 << b : 0;
+    cmask[w * m.max_deg + p] = (unsigned char)bits;
   }
-  __syncthreads();
-  int pself = 0;
-  for (int p = 0; p < deg; ++p)
-    if (m.adj[a0 + p] == n) pself = p;
-  const int L = NDOF * deg;
-  // entry (a, p, b) of the node's rows with the Dirichlet epilogue applied
-  auto entry = [&](int a, int p, int b) -> double {
-    double v = 0.0;
-    for (int k = 0; k < ninc; ++k) {
-      const int j = slot_dyn[k * deg + p];
-      if (j >= 0) {
-        const int64_t e = m.ne_elem[inc0 + k];
-        const int i = m.ne_loc[inc0 + k];
-        v += kin[e * W * W + (int64_t)(i * NDOF + a) * W + j * NDOF + b];
+  for (int t0 = 0; t0 < most; t0 += U) {
+    // (no branches around the loads: past the last element, or value, the
+    // last one is read again and not added)
+    int64_t e[U];
+    int il[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = inc0 + max(min(t0 + u, ninc - 1), 0);
+      e[u] = m.ne_elem[k];
+      il[u] = m.ne_loc[k];
+    }
+    double v[U][IR];
+    int at[U][IR];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < IR; ++r) {
+        const int q = min(l + r * LPN, NV - 1), j = q % W / NDOF;
+        v[u][r] = kin[e[u] * (W * W) + il[u] * NV + q];
+        at[u][r] = m.epos[(e[u] * NPE + il[u]) * NPE + j];
+        if (t0 + u == 0 && ninc > 0 && j == il[u]) tile.self[w] = at[u][r];
       }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < IR; ++r) {
+        const int q = l + r * LPN, a = q / W, col = q - a * W;
+        at[u][r] = t0 + u < ninc && q < NV ? a * L + at[u][r] * NDOF + col % NDOF : -1;
+      }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int r = 0; r < IR; ++r)
+        if (at[u][r] >= 0) acc[w * stride + at[u][r]] += v[u][r];
+      __syncthreads();
     }
-    const int64_t row = n * NDOF + a;
-    const int64_t col = (int64_t)m.adj[a0 + p] * NDOF + b;
-    if (con[row] || con[col]) v = (row == col) ? 1.0 : 0.0;
-    return v;
-  };
-  for (int q = tid; q < ND2 * deg; q += 64) {
-    const int a = q / L, rem = q - a * L, p = rem / NDOF, b = rem - p * NDOF;
-    const double v = entry(a, p, b);
-    if (v64) v64[vb + q] = v;
-    if (v32 && (p != pself || !diff32)) v32[vb + q] = (float)v;
-    if (p == pself) dblk[n * ND2 + a * NDOF + b] = v;
   }
-  // FP32 difference form: the diagonal block holds the FP64 row sums
-  if (v32 && diff32 && tid < ND2) {
-    const int a = tid / NDOF, b = tid - a * NDOF;
-    double r = 0.0;
-    for (int p = 0; p < deg; ++p) r += entry(a, p, b);
-    v32[vb + a * L + pself * NDOF + b] = (float)r;
-  }
+  __syncthreads();
+  tile_epilogue<NDOF, NW>(m, n0, acc, stride, cmask, tile, v64, v32, dblk, diff32);
 }
 
 // Sensitivities of lam^T K(p) u per element (see tfm_sensitivity in tfm.h):
@@ -1245,16 +1293,35 @@ int launch_assemble_elements(hipStream_t s, const tfm_mesh_t &m, const double *k
                              const uint8_t *con, double *v64, float *v32, double *dblk,
                              bool diff32) {
   if (m.n_nod == 0) return TFM_OK;
-  const size_t shm = (size_t)m.max_inc * m.max_deg;
-  TFM_REQUIRE(shm <= 48 * 1024, "node degree too large for the assembly kernel");
-  switch (m.ndof) {
-    case 1: hipLaunchKernelGGL(k_assemble_elements<1>, dim3((unsigned)m.n_nod), dim3(64), shm, s, m, k, con, v64, v32, dblk, (int)diff32); break;
-    case 2: hipLaunchKernelGGL(k_assemble_elements<2>, dim3((unsigned)m.n_nod), dim3(64), shm, s, m, k, con, v64, v32, dblk, (int)diff32); break;
-    case 3: hipLaunchKernelGGL(k_assemble_elements<3>, dim3((unsigned)m.n_nod), dim3(64), shm, s, m, k, con, v64, v32, dblk, (int)diff32); break;
-    default: TFM_REQUIRE(false, "ndof must be 1, 2 or 3");
+  TFM_REQUIRE((size_t)m.max_inc * m.max_deg <= 48 * 1024,
+              "node degree too large for the assembly kernel");
+  auto go = [&](auto kernel, int nw, int nd) -> int {
+    // at most 73 bytes per neighbour: 72 KB at the largest degree (990) that
+    // the bound above allows for 20 nodes per element
+    const size_t shm = (sizeof(double) * nd * nd + 1) * nw * (size_t)m.max_deg;
+    if (shm > 60 * 1024)
+      TFM_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((m.n_nod + nw - 1) / nw)), dim3(64), shm, s, m, k,
+                       con, v64, v32, dblk, (int)diff32);
+    TFM_CHECK_LAUNCH();
+    return TFM_OK;
+  };
+  auto by_ndof = [&](auto npe) -> int {
+    constexpr int N = decltype(npe)::value;
+    switch (m.ndof) {
+      case 1: return go(&k_assemble_elements<N, 1>, 64 / assemble_lanes(N, 1), 1);
+      case 2: return go(&k_assemble_elements<N, 2>, 64 / assemble_lanes(N, 2), 2);
+      case 3: return go(&k_assemble_elements<N, 3>, 64 / assemble_lanes(N, 3), 3);
+      default: TFM_REQUIRE(false, "ndof must be 1, 2 or 3");
+    }
+  };
+  switch (m.npe) {
+    case 4: return by_ndof(std::integral_constant<int, 4>{});
+    case 8: return by_ndof(std::integral_constant<int, 8>{});
+    case 20: return by_ndof(std::integral_constant<int, 20>{});
+    default: TFM_REQUIRE(false, "unsupported number of element nodes");
   }
-  TFM_CHECK_LAUNCH();
-  return TFM_OK;
 }
 
 int launch_gather(hipStream_t s, const tfm_mesh_t &m, const double *fe, double *F) {
