@@ -117,14 +117,22 @@ __global__ void k_inc_count(const int32_t *el, int64_t nent, int64_t n_nod, int3
   atomicAdd(&cnt[n], 1);
 }
 
-__global__ void k_inc_fill(const int32_t *el, int64_t nent, int npe, const int32_t *ptr,
+__global__ void k_inc_fill(const int32_t *el, int64_t nent, int npe, int64_t n_nod,
+                           const int32_t *ptr,
                            int32_t *cursor, int32_t *ne_elem, int32_t *ne_loc) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nent) return;
   const int32_t n = el[t];
+  if (n < 0 || n >= n_nod) return;  // refused by the caller (k_inc_count)
   const int32_t k = ptr[n] + atomicAdd(&cursor[n], 1);
   ne_elem[k] = (int32_t)(t / npe);
   ne_loc[k] = (int32_t)(t % npe);
+}
+
+// *most = max(*most, v): the atomic only where it would change something, so
+// that it does not queue every node on one address.
+__device__ __forceinline__ void raise(int32_t *most, int32_t v) {
+  if (__hip_atomic_load(most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(most, v);
 }
 
 // Incident elements of each node ascending (then by local index): a fixed
@@ -145,67 +153,168 @@ __global__ void k_inc_sort(int64_t n_nod, const int32_t *ptr, int32_t *ne_elem, 
     ne_elem[j + 1] = e;
     ne_loc[j + 1] = l;
   }
-  atomicMax(max_inc, b - a);
+  raise(max_inc, b - a);
 }
 
 // ---------------------------------------------------------------- adjacency
-// The sorted set of nodes that share an element with n (n included when it
-// belongs to an element), built by insertion with binary search in a local
-// list of at most PMAXDEG entries. Returns its size, -1 on overflow.
-__device__ int node_union(const int32_t *el, int npe, const int32_t *ne_ptr,
-                          const int32_t *ne_elem, int64_t n, int32_t *lst) {
-  int deg = 0;
-  for (int32_t k = ne_ptr[n]; k < ne_ptr[n + 1]; ++k) {
-    const int32_t *en = el + (int64_t)ne_elem[k] * npe;
-    for (int j = 0; j < npe; ++j) {
-      const int32_t c = en[j];
-      int lo = 0, hi = deg;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (lst[mid] < c) lo = mid + 1;
-        else hi = mid;
+// One wave per node. The node's candidates, the nodes of its incident elements
+// with repetitions (64 of Hexa1, 160 of Hexa2), are sorted in registers by a
+// bitonic network and their distinct values collected in LDS. An insertion
+// into a sorted list per thread, in scratch memory, took 290 us per pass on
+// 53x47x58 Hexa1 and 400 us on 13x15x11 Hexa2; this takes 89 and 29,
+// bound by the vector instructions of the sort. Filling needs 102 and 34 with epos
+// (357 and 410 before, with a search of adj in memory for every pair).
+constexpr int PROOM = 256;  // values that one sort holds
+// nodes (waves) per block: four took 84 and 106 us (one: 89 and 102) on Hexa1,
+// 46 and 35 (29 and 34) on Hexa2, where few nodes have the long lists
+constexpr int PNB = 1;
+constexpr int32_t PNONE = 0x7fffffff;
+
+// LDS accesses of a wave complete in order; the compiler must keep them so.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The smaller (or larger) of v and v of lane ^ J, by DPP within 16 lanes and
+// the row swaps across them: an LDS permutation for each of the 21 steps of 64
+// values was a third of the kernels' time.
+template <int J> __device__ __forceinline__ int32_t partner_min_max(int32_t v, bool smaller) {
+  int32_t a = v, b;
+  if constexpr (J == 32) {
+    const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = p[0];
+    b = p[1];
+  } else if constexpr (J == 16) {
+    const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    a = p[0];
+    b = p[1];
+  } else if constexpr (J == 4) {  // reversed in 8 lanes, then in 4
+    b = __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);
+    b = __builtin_amdgcn_update_dpp(0, b, 0x1B, 0xf, 0xf, true);
+  } else {
+    constexpr int CTRL = J == 1 ? 0xB1 : J == 2 ? 0x4E : 0x128;  // 8: rotated in 16
+    b = __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+  }
+  return smaller ? min(a, b) : max(a, b);
+}
+
+// One step of the network over R registers: the partners at distance J in
+// runs of K sorted alternately up and down.
+template <int R, int K, int J> __device__ __forceinline__ void sort_step(int32_t (&v)[R]) {
+  const int lane = threadIdx.x % 64;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = r * 64 + lane;
+    if constexpr (J >= 64) {
+      constexpr int D = J / 64;
+      if ((r & D) == 0) {
+        const int32_t lo = min(v[r], v[r + D]), hi = max(v[r], v[r + D]);
+        v[r] = (i & K) == 0 ? lo : hi;
+        v[r + D] = (i & K) == 0 ? hi : lo;
       }
-      if (lo < deg && lst[lo] == c) continue;
-      if (deg == PMAXDEG) return -1;
-      for (int q = deg; q > lo; --q) lst[q] = lst[q - 1];
-      lst[lo] = c;
-      ++deg;
+    } else {
+      v[r] = partner_min_max<J>(v[r], ((i & K) == 0) == ((i & J) == 0));
     }
   }
+  if constexpr (J > 1) sort_step<R, K, J / 2>(v);
+  else if constexpr (K < 64 * R) sort_step<R, 2 * K, K>(v);
+}
+
+// Ascending order of v[r] of lane l at index r * 64 + l.
+template <int R> __device__ __forceinline__ void wave_sort(int32_t (&v)[R]) {
+  sort_step<R, 2, 1>(v);
+}
+
+// Sorts v and puts its distinct values (PNONE apart) into lst; their number.
+template <int R> __device__ __forceinline__ int sort_distinct(int32_t (&v)[R], int32_t *lst) {
+  const int lane = threadIdx.x % 64;
+  wave_sort<R>(v);
+  int n = 0;
+  int32_t before = PNONE;  // the last value of the registers before
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    int32_t prev = __shfl_up(v[r], 1, 64);
+    if (lane == 0) prev = before;
+    before = __shfl(v[r], 63, 64);
+    const bool fresh = v[r] != PNONE && ((r == 0 && lane == 0) || v[r] != prev);
+    const unsigned long long mask = __ballot(fresh);
+    if (fresh) lst[n + __popcll(mask & ((1ull << lane) - 1ull))] = v[r];
+    n += __popcll(mask);
+  }
+  return n;
+}
+
+// The sorted set of nodes that share an element with a node (itself included
+// when it belongs to an element) in lst[PROOM]; its size, -1 beyond PMAXDEG.
+__device__ __forceinline__ int node_union(const int32_t *el, int npe, const int32_t *inc,
+                                          int ninc, int32_t *lst) {
+  const int lane = threadIdx.x % 64, C = ninc * npe;
+  auto candidate = [&](int i) -> int32_t {
+    return i < C ? el[(int64_t)inc[i / npe] * npe + i % npe] : PNONE;
+  };
+  int deg = 0;
+  if (C <= 64) {
+    int32_t v[1] = {candidate(lane)};
+    deg = sort_distinct<1>(v, lst);
+  } else if (C <= 128) {
+    int32_t v[2] = {candidate(lane), candidate(64 + lane)};
+    deg = sort_distinct<2>(v, lst);
+  } else {
+    // more than PROOM candidates are merged into the list piece by piece
+    for (int c = 0; c < C; ) {
+      int32_t v[PROOM / 64];
+#pragma unroll
+      for (int r = 0; r < PROOM / 64; ++r) {
+        const int i = r * 64 + lane;
+        v[r] = i < deg ? lst[i] : candidate(c + i - deg);
+      }
+      c += PROOM - deg;
+      wave_sync();
+      deg = sort_distinct<PROOM / 64>(v, lst);
+      wave_sync();
+      if (deg > PMAXDEG) return -1;
+    }
+  }
+  wave_sync();
   return deg;
 }
 
 // deg[n] and the value count of n's rows (deg * ndof^2, or ndof for a node
 // of no element)
-__global__ void k_adj_count(const int32_t *el, int npe, int64_t n_nod, const int32_t *ne_ptr,
-                            const int32_t *ne_elem, int ndof, int32_t *deg, int32_t *nval,
-                            int32_t *max_deg, int32_t *bad) {
-  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(64 * PNB) k_adj_count(const int32_t *el, int npe,
+                                                  int64_t n_nod, const int32_t *ne_ptr,
+                                                  const int32_t *ne_elem, int ndof, int32_t *deg, int32_t *nval,
+                                                  int32_t *max_deg, int32_t *bad) {
+  __shared__ int32_t lists[PNB][PROOM];
+  int32_t *lst = lists[threadIdx.x / 64];
+  const int64_t n = xcd_block() * PNB + threadIdx.x / 64;
   if (n >= n_nod) return;
-  int32_t lst[PMAXDEG];
-  const int d = node_union(el, npe, ne_ptr, ne_elem, n, lst);
-  if (d < 0) {
-    *bad = 2;
-    deg[n] = 0;
-    nval[n] = ndof;
-    return;
-  }
-  deg[n] = d;
+  const int32_t i0 = ne_ptr[n];
+  const int d = node_union(el, npe, ne_elem + i0, ne_ptr[n + 1] - i0, lst);
+  if (threadIdx.x % 64 != 0) return;
+  if (d < 0) *bad = 2;
+  deg[n] = d > 0 ? d : 0;
   nval[n] = d > 0 ? d * ndof * ndof : ndof;
-  atomicMax(max_deg, d);
+  raise(max_deg, d);
 }
 
 // adj (and the 16-bit offsets adj - n when adj16 is given; *wide is set if
-// some offset does not fit)
-__global__ void k_adj_fill(const int32_t *el, int npe, int64_t n_nod, const int32_t *ne_ptr,
-                           const int32_t *ne_elem, const int32_t *adj_ptr, int32_t *adj,
-                           int16_t *adj16, int32_t *wide) {
-  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// some offset does not fit), and epos[e][i][j], the position of element node j
+// in the adjacency of node i, for the incidences (e, i) of the node
+__global__ void __launch_bounds__(64 * PNB) k_adj_fill(const int32_t *el, int npe,
+                                                 int64_t n_nod, const int32_t *ne_ptr,
+                                                 const int32_t *ne_elem, const int32_t *adj_ptr, int32_t *adj,
+                                                 int16_t *adj16, int32_t *wide, uint16_t *epos) {
+  __shared__ int32_t lists[PNB][PROOM];
+  int32_t *lst = lists[threadIdx.x / 64];
+  const int lane = threadIdx.x % 64;
+  const int64_t n = xcd_block() * PNB + threadIdx.x / 64;
   if (n >= n_nod) return;
-  int32_t lst[PMAXDEG];
-  const int d = node_union(el, npe, ne_ptr, ne_elem, n, lst);
-  const int32_t a0 = adj_ptr[n];
-  for (int q = 0; q < d; ++q) {
+  const int32_t i0 = ne_ptr[n], ninc = ne_ptr[n + 1] - i0, a0 = adj_ptr[n];
+  const int d = node_union(el, npe, ne_elem + i0, ninc, lst);
+  for (int q = lane; q < d; q += 64) {
     adj[a0 + q] = lst[q];
     if (adj16) {
       const int64_t delta = (int64_t)lst[q] - n;
@@ -213,24 +322,19 @@ __global__ void k_adj_fill(const int32_t *el, int npe, int64_t n_nod, const int3
       adj16[a0 + q] = (int16_t)delta;
     }
   }
-}
-
-// epos[e][i][j]: position of element node j in the adjacency of node i
-__global__ void k_epos(const int32_t *el, int64_t n_elem, int npe, const int32_t *adj_ptr,
-                       const int32_t *adj, uint16_t *epos) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n_elem * npe * npe) return;
-  const int64_t e = t / (npe * npe);
-  const int r = (int)(t - e * npe * npe), i = r / npe, j = r - i * npe;
-  const int32_t ni = el[e * npe + i], nj = el[e * npe + j];
-  int lo = adj_ptr[ni], hi = adj_ptr[ni + 1];
-  const int base = lo;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (adj[mid] < nj) lo = mid + 1;
-    else hi = mid;
+  for (int t = lane; t < ninc * npe; t += 64) {
+    const int k = t / npe, j = t - k * npe;
+    const int64_t e = ne_elem[i0 + k];
+    const int32_t c = el[e * npe + j];
+    int lo = 0, hi = d;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (lst[mid] < c) lo = mid + 1;
+      else hi = mid;
+    }
+    for (int i = 0; i < npe; ++i)  // (an element may name the node twice)
+      if (el[e * npe + i] == n) epos[(e * npe + i) * npe + j] = (uint16_t)lo;
   }
-  epos[t] = (uint16_t)(lo - base);
 }
 
 }  // namespace
@@ -263,16 +367,17 @@ extern "C" int tfm_pattern_device_count(tfm_stream_t stream, const int32_t *elem
   if (rc != TFM_OK) return rc;
   if (nent > 0) {
     hipLaunchKernelGGL(k_inc_fill, dim3(pblocks(nent)), dim3(PB), 0, s, elements, nent, npe,
-                       (const int32_t *)ne_ptr, cursor, ne_elem, ne_loc);
+                       n_nod, (const int32_t *)ne_ptr, cursor, ne_elem, ne_loc);
     TFM_CHECK_LAUNCH();
   }
   if (n_nod > 0) {
     hipLaunchKernelGGL(k_inc_sort, dim3(pblocks(n_nod)), dim3(PB), 0, s, n_nod,
                        (const int32_t *)ne_ptr, ne_elem, ne_loc, flags + 1);
     TFM_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_adj_count, dim3(pblocks(n_nod, 64)), dim3(64), 0, s, elements, (int)npe,
-                       n_nod, (const int32_t *)ne_ptr, (const int32_t *)ne_elem, (int)ndof, cnt,
-                       nval, flags + 2, flags);
+    hipLaunchKernelGGL(k_adj_count, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s,
+                       elements, (int)npe, n_nod, (const int32_t *)ne_ptr,
+                       (const int32_t *)ne_elem, (int)ndof, cnt, nval,
+                       flags + 2, flags);
     TFM_CHECK_LAUNCH();
   }
   rc = pscan<int32_t>(s, cnt, n_nod, bsum32, adj_ptr);
@@ -304,14 +409,9 @@ extern "C" int tfm_pattern_device_fill(tfm_stream_t stream, const int32_t *eleme
   hipStream_t s = (hipStream_t)stream;
   TFM_CHECK_HIP(hipMemsetAsync(work, 0, sizeof(int32_t), s));
   if (n_nod > 0) {
-    hipLaunchKernelGGL(k_adj_fill, dim3(pblocks(n_nod, 64)), dim3(64), 0, s, elements, (int)npe,
-                       n_nod, ne_ptr, ne_elem, adj_ptr, adj, adj16, work);
-    TFM_CHECK_LAUNCH();
-  }
-  const int64_t ne = n_elem * npe * npe;
-  if (ne > 0) {
-    hipLaunchKernelGGL(k_epos, dim3(pblocks(ne)), dim3(PB), 0, s, elements, n_elem, (int)npe,
-                       adj_ptr, (const int32_t *)adj, epos);
+    hipLaunchKernelGGL(k_adj_fill, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s,
+                       elements, (int)npe, n_nod, ne_ptr,
+                       ne_elem, adj_ptr, adj, adj16, work, epos);
     TFM_CHECK_LAUNCH();
   }
   int32_t wide = 0;
