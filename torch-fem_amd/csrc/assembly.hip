@@ -59,73 +59,107 @@ __device__ __forceinline__ void bcol(const double (&Ji)[E::DIM][E::DIM], int g, 
 }
 
 // ========================================================= pattern expansion
-// Row pointer of DOF row (n, a) of the node-block layout.
-__device__ __forceinline__ int64_t row_start(const tfm_mesh_t &m, int64_t n, int a, int deg) {
-  return m.val_ptr[n] + (deg > 0 ? (int64_t)a * m.ndof * deg : a);
-}
-
-__global__ void k_pattern_rows(tfm_mesh_t m, int64_t *rows, int64_t *cols, int64_t *rowptr,
-                               int32_t *diag_map) {
-  const int64_t n = xcd_block();
-  const int nd = m.ndof;
+// A wave per node, four to a block. Bound by writing rows and cols: 573 MB of
+// 53x47x58 Hexa1 in 160 us (284 with a block of 256 per node, every thread of
+// which searched the diagonal).
+template <int ND>
+__global__ void __launch_bounds__(256) k_pattern_rows(tfm_mesh_t m, int64_t *rows, int64_t *cols,
+                                                      int64_t *rowptr, int32_t *diag_map) {
+  const int64_t n = xcd_block() * 4 + threadIdx.x / 64;
+  const int lane = threadIdx.x % 64;
+  if (n >= m.n_nod) return;
   const int a0 = m.adj_ptr[n];
   const int deg = m.adj_ptr[n + 1] - a0;
-  int pself = 0;
-  for (int p = 0; p < deg; ++p)
-    if (m.adj[a0 + p] == n) pself = p;
-  if (threadIdx.x < nd) {
-    const int a = threadIdx.x;
-    const int64_t rs = row_start(m, n, a, deg);
-    if (rowptr) {
-      rowptr[n * nd + a] = rs;
-      if (n == m.n_nod - 1 && a == nd - 1) rowptr[m.n_nod * nd] = m.nnz;
+  const int64_t v0 = m.val_ptr[n];
+  const int L = ND * deg;
+  if (lane < ND && rowptr) {
+    rowptr[n * ND + lane] = v0 + (deg > 0 ? lane * L : lane);
+    if (n == m.n_nod - 1 && lane == ND - 1) rowptr[m.n_nod * ND] = m.nnz;
+  }
+  if (diag_map) {
+    if (deg == 0) {
+      if (lane < ND) diag_map[n * ND + lane] = (int32_t)(v0 + lane);
+    } else {
+      for (int p = lane; p < deg; p += 64)
+        if (m.adj[a0 + p] == n)
+          for (int a = 0; a < ND; ++a)
+            diag_map[n * ND + a] = (int32_t)(v0 + a * L + p * ND + a);
     }
-    if (diag_map) diag_map[n * nd + a] = (int32_t)(deg > 0 ? rs + (int64_t)pself * nd + a : rs);
   }
   if (!rows && !cols) return;
-  if (deg == 0) {
-    if (threadIdx.x < nd) {
-      const int64_t q = m.val_ptr[n] + threadIdx.x;
-      if (rows) rows[q] = n * nd + threadIdx.x;
-      if (cols) cols[q] = n * nd + threadIdx.x;
+  const int total = deg > 0 ? ND * L : ND;
+  for (int q = lane; q < total; q += 64) {
+    int a = q;
+    int64_t col = n * ND + q;
+    if (deg > 0) {
+      int rem = q;  // q = a L + rem
+      a = 0;
+      for (int k = 1; k < ND; ++k)
+        if (rem >= L) {
+          rem -= L;
+          ++a;
+        }
+      const int p = rem / ND;
+      col = (int64_t)m.adj[a0 + p] * ND + (rem - p * ND);
     }
-    return;
-  }
-  const int L = nd * deg;
-  for (int q = threadIdx.x; q < nd * L; q += blockDim.x) {
-    const int a = q / L, rem = q - a * L, p = rem / nd, b = rem - p * nd;
-    const int64_t o = m.val_ptr[n] + q;
-    if (rows) rows[o] = n * nd + a;
-    if (cols) cols[o] = (int64_t)m.adj[a0 + p] * nd + b;
+    if (rows) rows[v0 + q] = n * ND + a;
+    if (cols) cols[v0 + q] = col;
   }
 }
 
-// k_map[e, i*nd+a, j*nd+b] = slot of (row n_i*nd+a, col n_j*nd+b) (base.py:94-104)
-__global__ void k_pattern_kmap(tfm_mesh_t m, int32_t *k_map) {
-  const int64_t e = xcd_block();
-  const int npe = m.npe, nd = m.ndof, W = npe * nd;
-  for (int t = threadIdx.x; t < W * W; t += blockDim.x) {
-    const int r = t / W, c = t - r * W;
-    const int i = r / nd, a = r - i * nd, j = c / nd, b = c - j * nd;
-    const int64_t ni = m.elements[e * npe + i];
-    const int deg = m.adj_ptr[ni + 1] - m.adj_ptr[ni];
-    const int pos = m.epos[(e * npe + i) * npe + j];
-    k_map[e * W * W + t] = (int32_t)(row_start(m, ni, a, deg) + (int64_t)pos * nd + b);
+// k_map[e, i*nd+a, j*nd+b] = slot of (row n_i*nd+a, col n_j*nd+b) (base.py:94-104).
+// The row starts of the nodes of EB elements and their slots in LDS; the map
+// leaves in consecutive words, its bound: 333 MB of 53x47x58 Hexa1 in 122 us (242
+// with all of it looked up per entry; 223 with divisions by run-time widths).
+template <int NPE, int ND>
+__global__ void __launch_bounds__(256) k_pattern_kmap(tfm_mesh_t m, int32_t *k_map) {
+  constexpr int EB = NPE <= 8 ? 4 : 1, W = NPE * ND, W2 = W * W, NP2 = NPE * NPE;
+  __shared__ int start[EB * NPE], len[EB * NPE], pos[EB * NP2];
+  const int64_t e0 = xcd_block() * EB;
+  const int ne = (int)(m.n_elem - e0 < EB ? m.n_elem - e0 : EB);
+  for (int t = threadIdx.x; t < ne * NPE; t += 256) {
+    const int64_t n = m.elements[e0 * NPE + t];
+    start[t] = (int)m.val_ptr[n];
+    len[t] = ND * (m.adj_ptr[n + 1] - m.adj_ptr[n]);
   }
+  for (int t = threadIdx.x; t < ne * NP2; t += 256) pos[t] = m.epos[e0 * NP2 + t];
+  __syncthreads();
+  for (int t = threadIdx.x; t < ne * W2; t += 256) {
+    const int k = t / W2, q = t - k * W2, r = q / W, c = q - r * W;
+    const int i = r / ND, a = r - i * ND, j = c / ND, b = c - j * ND;
+    k_map[e0 * W2 + t] = start[k * NPE + i] + a * len[k * NPE + i] + pos[k * NP2 + i * NPE + j] * ND + b;
+  }
+}
+
+template <int ND>
+static int pattern_expand(hipStream_t s, const tfm_mesh_t &m, int64_t *rows, int64_t *cols,
+                          int64_t *rowptr, int32_t *k_map, int32_t *diag_map) {
+  if (rows || cols || rowptr || diag_map) {
+    hipLaunchKernelGGL(k_pattern_rows<ND>, dim3((unsigned)((m.n_nod + 3) / 4)), dim3(256), 0, s, m,
+                       rows, cols, rowptr, diag_map);
+    TFM_CHECK_LAUNCH();
+  }
+  if (k_map && m.n_elem > 0) {
+    const unsigned by4 = (unsigned)((m.n_elem + 3) / 4), by1 = (unsigned)m.n_elem;
+    switch (m.npe) {
+      case 4: hipLaunchKernelGGL((k_pattern_kmap<4, ND>), dim3(by4), dim3(256), 0, s, m, k_map); break;
+      case 8: hipLaunchKernelGGL((k_pattern_kmap<8, ND>), dim3(by4), dim3(256), 0, s, m, k_map); break;
+      case 20: hipLaunchKernelGGL((k_pattern_kmap<20, ND>), dim3(by1), dim3(256), 0, s, m, k_map); break;
+      default: TFM_REQUIRE(false, "unsupported number of element nodes");
+    }
+    TFM_CHECK_LAUNCH();
+  }
+  return TFM_OK;
 }
 
 int launch_pattern_expand(hipStream_t s, const tfm_mesh_t &m, int64_t *rows, int64_t *cols,
                           int64_t *rowptr, int32_t *k_map, int32_t *diag_map) {
-  if (rows || cols || rowptr || diag_map) {
-    hipLaunchKernelGGL(k_pattern_rows, dim3((unsigned)m.n_nod), dim3(256), 0, s, m, rows, cols,
-                       rowptr, diag_map);
-    TFM_CHECK_LAUNCH();
+  switch (m.ndof) {
+    case 1: return pattern_expand<1>(s, m, rows, cols, rowptr, k_map, diag_map);
+    case 2: return pattern_expand<2>(s, m, rows, cols, rowptr, k_map, diag_map);
+    case 3: return pattern_expand<3>(s, m, rows, cols, rowptr, k_map, diag_map);
+    default: TFM_REQUIRE(false, "ndof must be 1, 2 or 3");
   }
-  if (k_map && m.n_elem > 0) {
-    hipLaunchKernelGGL(k_pattern_kmap, dim3((unsigned)m.n_elem), dim3(256), 0, s, m, k_map);
-    TFM_CHECK_LAUNCH();
-  }
-  return TFM_OK;
 }
 
 // ========================================================= element matrices

@@ -152,12 +152,15 @@ class DevicePattern:
         return L.stream_of(self.device)
 
     def expand(self, rows=True, cols=True, rowptr=False, k_map=False, diag_map=False):
-        """The reference's index arrays, expanded on the device."""
+        """The reference's index arrays, expanded on the device. Rows and
+        columns asked for together lie one after the other, as glob_idx."""
         dev = self.device
         W = self.npe * self.ndof
+        idx = torch.empty(int(rows) + int(cols), self.nnz, dtype=torch.int64, device=dev)
         out = {
-            "rows": torch.empty(self.nnz, dtype=torch.int64, device=dev) if rows else None,
-            "cols": torch.empty(self.nnz, dtype=torch.int64, device=dev) if cols else None,
+            "glob_idx": idx if rows and cols else None,
+            "rows": idx[0] if rows else None,
+            "cols": idx[-1] if cols else None,
             "rowptr": torch.empty(self.n_dofs + 1, dtype=torch.int64, device=dev) if rowptr else None,
             "k_map": torch.empty(self.n_elem * W * W, dtype=torch.int32, device=dev) if k_map else None,
             "diag_map": torch.empty(self.n_dofs, dtype=torch.int32, device=dev) if diag_map else None,

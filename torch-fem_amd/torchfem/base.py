@@ -330,8 +330,7 @@ class FEM(ABC):
     @cached_property
     def glob_idx(self) -> Tensor:
         """Row/column indices [2, nnz] int64 of the pattern (base.py:112-117)."""
-        e = self._pattern.expand(rows=True, cols=True)
-        return torch.stack([e["rows"], e["cols"]])
+        return self._pattern.expand(rows=True, cols=True)["glob_idx"]
 
     @cached_property
     def k_map(self) -> Tensor:
