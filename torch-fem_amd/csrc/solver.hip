@@ -240,16 +240,16 @@ __device__ __forceinline__ void node_product_at(const tfm_mesh_t &m, const T *__
   }
 }
 
-// FP32 with four or more rhs: the team's ND*NRP sums per lane are reduced
-// through LDS instead of a butterfly (48 values over 5 butterfly steps cost
-// 240 lane exchanges per node for 16 rhs). Each lane writes its sums as one
+// FP32 with four or eight rhs: the team's ND*NRP sums per lane are reduced
+// through LDS instead of a butterfly (24 values over 5 butterfly steps cost 120
+// lane exchanges per node). Each lane writes its sums as one
 // row of a TL x (ND*NRP) table (padded to an odd row length, so neither
 // the row writes nor the column reads conflict), then lane l adds column
 // e = l + k*TL over the TL rows in order. outv[k] is entry e of the node's
 // outputs. The team is inside one wave, whose LDS accesses complete in
 // order, so only the compiler has to be kept from reordering them.
 template <typename T, int TL, int NRP> constexpr bool lds_reduce() {
-  return sizeof(T) == 4 && NRP >= 4 && TL < 64;
+  return sizeof(T) == 4 && (NRP == 4 || NRP == 8) && TL < 64;
 }
 
 template <typename T, int ND, int TL, int NRP, bool D16>
@@ -288,26 +288,84 @@ __device__ __forceinline__ void node_product(const tfm_mesh_t &m, const T *__res
   node_product_at<T, ND, TL, NRP, D16>(m, val, x, n, node_ptr(m, n), lane, acc);
 }
 
-// Several right-hand sides (NRP >= 4): one 64-lane wave per node. Lane
-// l = q*NRP + 4*g + t (t < 4) works on rhs group g (rhs 4g..4g+3) and on the
-// neighbour blocks p = s, s + S, ... of slice s = 4*q + t (S = 256/NRP
-// slices). The lanes of one slice load the same block rows (one transaction
-// serves them) and the four rhs of their group at the neighbour in one
-// 16-byte load (contiguous in the interleaved layout). A butterfly over the
-// slices (lane offsets 1, 2 and multiples of NRP) leaves the ND x 4 sums of
-// group g in every lane of the group, so lane l holds entry e = l of the
-// node's ND*NRP outputs (rhs l % NRP). ND*4 accumulators per lane instead of
-// ND*NRP keep the kernel's occupancy.
+// Several right-hand sides, FP64: one 64-lane wave per node, G = NRP / 4 lanes
+// per neighbour block. Lane l works on rhs 4 g .. 4 g + 3 with g = l % G and on the
+// blocks p = s, s + S, ... of slice s = l / G (S = 64 / G slices): the G lanes
+// of a block read the NRP values of x at the neighbour as one run, and its rows
+// from the same addresses. With the lanes of a block 4 apart, where the L1
+// serves their lines one by one, the product of Hexa2 21x19x23 with 16 rhs
+// took 155 us, now 118.
+// The sums over the slices leave lane l with entry (a, rhs) = (l / NRP,
+// rg_rhs(l)) of the node's ND x NRP outputs, by exchanges that halve the values
+// a lane carries at each step where the lane's bit selects a component or a
+// rhs, and by plain butterflies over the bits that select neither.
 template <int TL, int NRP> constexpr bool rhs_lanes() { return TL == 64 && NRP >= 4; }
 
+template <int NRP> __device__ __forceinline__ int rg_rhs(int lane) {
+  constexpr int G = NRP / 4;
+  return 4 * (lane % G) + lane % NRP / G;
+}
+// the lane, of those with lane / NRP = 0, that holds rhs r
+template <int NRP> __device__ __forceinline__ int rg_lane(int r) {
+  return r % 4 * (NRP / 4) + r / 4;
+}
+
+// x of lane ^ OFF
+template <int OFF> __device__ __forceinline__ int lane_xor(int x) {
+  if constexpr (OFF == 4) {  // reversed in 8 lanes, then in 4
+    x = __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true);
+    return __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xf, 0xf, true);
+  } else if constexpr (OFF < 16) {
+    constexpr int CTRL = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : 0x128;  // 8: rotated in 16
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+  } else {
+    return __shfl_xor(x, OFF, 64);
+  }
+}
+template <int OFF> __device__ __forceinline__ float lane_xor(float x) {
+  return __int_as_float(lane_xor<OFF>(__float_as_int(x)));
+}
+template <int OFF> __device__ __forceinline__ double lane_xor(double x) {
+  return __hiloint2double(lane_xor<OFF>(__double2hiint(x)), lane_xor<OFF>(__double2loint(x)));
+}
+
+// v0 summed over the lane and lane ^ OFF in the lanes whose bit OFF is clear,
+// v1 in the others.
+template <int OFF, typename T> __device__ __forceinline__ T halve(T v0, T v1, int lane) {
+  if constexpr (OFF >= 16) {  // a row swap puts each lane's two terms into place
+    constexpr int NWORD = sizeof(T) / 4;
+    int a[NWORD], b[NWORD];
+    __builtin_memcpy(a, &v0, sizeof(T));
+    __builtin_memcpy(b, &v1, sizeof(T));
+#pragma unroll
+    for (int k = 0; k < NWORD; ++k) {
+      if constexpr (OFF == 16) {
+        const auto p = __builtin_amdgcn_permlane16_swap(a[k], b[k], false, false);
+        a[k] = p[0];
+        b[k] = p[1];
+      } else {
+        const auto p = __builtin_amdgcn_permlane32_swap(a[k], b[k], false, false);
+        a[k] = p[0];
+        b[k] = p[1];
+      }
+    }
+    __builtin_memcpy(&v0, a, sizeof(T));
+    __builtin_memcpy(&v1, b, sizeof(T));
+    return v0 + v1;
+  }
+  const bool up = (lane & OFF) != 0;
+  const T keep = up ? v1 : v0, send = up ? v0 : v1;
+  return keep + lane_xor<OFF>(send);
+}
+
 template <typename T, int ND, int NRP, bool D16>
-__device__ __forceinline__ void node_product_mr(const tfm_mesh_t &m, const T *__restrict__ val,
-                                                const T *__restrict__ x, int64_t n,
-                                                const NodePtr &np, int lane, T (&acc)[ND][4]) {
-  constexpr int S = 256 / NRP;
-  const int j = lane % NRP, g = j / 4;
-  const int sl = (lane / NRP) * 4 + (j % 4);
+__device__ __forceinline__ T node_product_rg(const tfm_mesh_t &m, const T *__restrict__ val,
+                                             const T *__restrict__ x, int64_t n,
+                                             const NodePtr &np, int lane) {
+  constexpr int G = NRP / 4, S = 64 / G;
+  const int g = lane % G, sl = lane / G;
   auto nbr = [&](int k) -> int64_t { return D16 ? n + (int64_t)m.adj16[k] : (int64_t)m.adj[k]; };
+  T acc[ND][4];
 #pragma unroll
   for (int a = 0; a < ND; ++a)
 #pragma unroll
@@ -341,30 +399,114 @@ __device__ __forceinline__ void node_product_mr(const tfm_mesh_t &m, const T *__
 #pragma unroll
       for (int t = 0; t < 4; ++t) acc[a][t] = vn[a] * x[(n * ND + a) * NRP + 4 * g + t];
   }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    if (off >= 4 && off < NRP) continue;  // these offsets change the rhs group
+  // bits of the lane: g (G lanes), t (4 G), a (16 G), the rest
+  if constexpr (16 * G < 32)
 #pragma unroll
     for (int a = 0; a < ND; ++a)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) acc[a][t] += __shfl_xor(acc[a][t], off, 64);
+      for (int t = 0; t < 4; ++t) acc[a][t] += lane_xor<16>(acc[a][t]);
+  if constexpr (16 * G < 64)
+#pragma unroll
+    for (int a = 0; a < ND; ++a)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[a][t] += lane_xor<32>(acc[a][t]);
+  T w[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const T v1 = ND > 1 ? acc[ND > 1 ? 1 : 0][t] : T(0), v2 = ND > 2 ? acc[ND > 2 ? 2 : 0][t] : T(0);
+    w[t] = halve<4 * G>(halve<8 * G>(acc[0][t], v2, lane), halve<8 * G>(v1, T(0), lane), lane);
+  }
+  return halve<G>(halve<2 * G>(w[0], w[2], lane), halve<2 * G>(w[1], w[3], lane), lane);
+}
+
+// Sixteen right-hand sides, FP32: a team of TL lanes per node, a neighbour block
+// per lane for its rows and its index, and four lanes per block for x. Lane l
+// loads the rows of block p = l, l + TL, ...; then the four lanes of a quad take
+// their blocks one after the other, each lane rhs 4 g .. 4 g + 3 (g = l % 4)
+// with the block's rows broadcast to it by DPP. x at a neighbour is thus read
+// as one run of 64 bytes and the rows once. Lanes that read all of x for a block
+// of their own touch a line for every 16 bytes: 51 us on Hexa2 21x19x23 (86 MB
+// of values), now 44; a conjugate-gradient solve of Hexa1 30x28x33 81 and 74 ms.
+// A wave per node as in FP64 took 55 us. With eight rhs, pairs of lanes were as
+// fast as a lane per block (51 and 49 ms on Hexa1 30x28x33), which is kept.
+// The sums over the quads leave lane l with entries e = l / 16 * 16 +
+// rg_rhs(l) + k TL of the node's ND x 16 outputs (see node_product_rg).
+template <typename T, int TL, int NRP> constexpr bool rhs_quads() {
+  return sizeof(T) == 4 && NRP == 16 && TL < 64;
+}
+
+// x of lane I of the quad
+template <int I> __device__ __forceinline__ int quad_lane(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, I * 0x55, 0xf, 0xf, true);
+}
+
+template <int ND, int TL, int NRP, bool D16>
+__device__ __forceinline__ void node_product_quads(const tfm_mesh_t &m,
+                                                   const float *__restrict__ val,
+                                                   const float *__restrict__ x, int64_t n,
+                                                   const NodePtr &np, int lane,
+                                                   float (&out)[(ND * NRP + TL - 1) / TL]) {
+  constexpr int G = 4;
+  static_assert(NRP == 4 * G && (TL == 16 || TL == 32), "team width");
+  const int g = lane % G;
+  float acc[ND][4];
+#pragma unroll
+  for (int a = 0; a < ND; ++a)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[a][t] = 0.0f;
+  const float *vn = val + np.v0;
+  for (int p0 = 0; p0 < np.deg; p0 += TL) {
+    const int p = p0 + lane;
+    Vec<float, ND> rows[ND]{};  // past the last block: zeros times the node's own x
+    int col = (int)n;
+    if (p < np.deg) {
+      col = D16 ? (int)n + (int)m.adj16[np.a0 + p] : m.adj[np.a0 + p];
+#pragma unroll
+      for (int a = 0; a < ND; ++a) rows[a] = ldv<float, ND>(vn + a * ND * np.deg + p * ND);
+    }
+    auto part = [&](auto index) {
+      constexpr int I = decltype(index)::value;
+      const int64_t c = quad_lane<I>(col);
+      Vec<float, 4> xv[ND];
+#pragma unroll
+      for (int b = 0; b < ND; ++b) xv[b] = ldv<float, 4>(x + (c * ND + b) * NRP + 4 * g);
+#pragma unroll
+      for (int a = 0; a < ND; ++a)
+#pragma unroll
+        for (int b = 0; b < ND; ++b) {
+          const float k = __int_as_float(quad_lane<I>(__float_as_int(rows[a].v[b])));
+#pragma unroll
+          for (int t = 0; t < 4; ++t) acc[a][t] += k * xv[b].v[t];
+        }
+    };
+    part(std::integral_constant<int, 0>{});
+    part(std::integral_constant<int, 1>{});
+    part(std::integral_constant<int, 2>{});
+    part(std::integral_constant<int, 3>{});
+  }
+  if (np.deg == 0 && lane < G) {  // orphan node: only its diagonal is stored
+#pragma unroll
+    for (int a = 0; a < ND; ++a)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[a][t] = vn[a] * x[(n * ND + a) * NRP + 4 * g + t];
+  }
+  auto by_rhs = [&](const float (&w)[4]) -> float {
+    return halve<G>(halve<2 * G>(w[0], w[2], lane), halve<2 * G>(w[1], w[3], lane), lane);
+  };
+  if constexpr (TL == 16) {
+#pragma unroll
+    for (int a = 0; a < ND; ++a) out[a] = by_rhs(acc[a]);
+  } else {  // bit 16 of the lane tells the components 0 and 1 apart
+    float w[2][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      w[0][t] = halve<16>(acc[0][t], ND > 1 ? acc[ND > 1 ? 1 : 0][t] : 0.0f, lane);
+      w[1][t] = halve<16>(acc[ND - 1][t], 0.0f, lane);
+    }
+    out[0] = by_rhs(w[0]);
+    if constexpr (ND == 3) out[1] = by_rhs(w[1]);
   }
 }
-
-// Entry e = a*NRP + r of a node's outputs from the group sums of the lane
-// that holds rhs r (a select chain, no indexed registers).
-template <typename T, int ND, int NRP>
-__device__ __forceinline__ T pick_entry(const T (&acc)[ND][4], int e) {
-  const int a = e / NRP, t = e % 4;
-  T w = acc[0][0];
-#pragma unroll
-  for (int aa = 0; aa < ND; ++aa)
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
-      if (aa == a && tt == t) w = acc[aa][tt];
-  return w;
-}
-
 
 // y = K x over the node blocks (every right-hand side of the interleaved x).
 template <typename T, int ND, int TL, int NRP, bool D16>
@@ -374,9 +516,16 @@ __global__ void __launch_bounds__(BS) k_spmv(tfm_mesh_t m, const T *__restrict__
   const int lane = threadIdx.x % TL, team = threadIdx.x / TL;
   for (int64_t n = (int64_t)blockIdx.x * TPB + team; n < m.n_nod; n += (int64_t)gridDim.x * TPB) {
     if constexpr (rhs_lanes<TL, NRP>()) {
-      T am[ND][4];
-      node_product_mr<T, ND, NRP, D16>(m, val, x, n, node_ptr(m, n), lane, am);
-      if (lane < ND * NRP) y[n * ND * NRP + lane] = pick_entry<T, ND, NRP>(am, lane);
+      const T w = node_product_rg<T, ND, NRP, D16>(m, val, x, n, node_ptr(m, n), lane);
+      if (lane < ND * NRP) y[n * ND * NRP + lane / NRP * NRP + rg_rhs<NRP>(lane)] = w;
+    } else if constexpr (rhs_quads<T, TL, NRP>()) {
+      constexpr int KE = (ND * NRP + TL - 1) / TL;
+      T outv[KE];
+      node_product_quads<ND, TL, NRP, D16>(m, val, x, n, node_ptr(m, n), lane, outv);
+      const int e0 = lane / NRP * NRP + rg_rhs<NRP>(lane);
+#pragma unroll
+      for (int k = 0; k < KE; ++k)
+        if (e0 + k * TL < ND * NRP) y[n * ND * NRP + e0 + k * TL] = outv[k];
     } else if constexpr (lds_reduce<T, TL, NRP>()) {
       constexpr int KE = (ND * NRP + TL - 1) / TL;
       T outv[KE];
@@ -586,10 +735,15 @@ __device__ __forceinline__ void spmv_dir_body(const tfm_mesh_t &m, const T *__re
     if (!dir_prologue<NRP>(it, part_in, n_in, st, sh, tot, beta, live, ended)) return;
   }
   // lane l updates the elements e = l, l + TL, ... of the node's ND*NRP
-  // (offset e from the node's first entry); they all belong to rhs l % NRP
+  // (offset e from the node's first entry); they all belong to rhs l % NRP.
+  // With the rhs across lanes it updates the one that its product leaves it.
   constexpr int NE = ND * NRP, KE = (NE + TL - 1) / TL;
-  const T b = (T)beta[lane % NRP];
-  const bool lv = live[lane % NRP] != 0;
+  constexpr bool RG = rhs_lanes<TL, NRP>(), QUADS = rhs_quads<T, TL, NRP>();
+  int rhs = lane % NRP;
+  if constexpr (RG || QUADS) rhs = rg_rhs<NRP>(lane);
+  const int e0 = lane / NRP * NRP + rhs;
+  const T b = (T)beta[rhs];
+  const bool lv = live[rhs] != 0;
   double dot = 0.0;
   for (; n < n_end; n += stride) {
     NodePtr cur;
@@ -603,7 +757,7 @@ __device__ __forceinline__ void spmv_dir_body(const tfm_mesh_t &m, const T *__re
     T up[KE], pp[KE], sp[KE];  // issued with the SpMV loads, used after it
 #pragma unroll
     for (int k = 0; k < KE; ++k) {
-      const int e = lane + k * TL;
+      const int e = e0 + k * TL;
       if (lv && e < NE) {
         up[k] = u[nb + e];
         pp[k] = p[nb + e];
@@ -611,21 +765,23 @@ __device__ __forceinline__ void spmv_dir_body(const tfm_mesh_t &m, const T *__re
       }
     }
     acc_t<T, NRP> acc[ND][NRP];
-    T am[ND][4], outv[KE];
-    if constexpr (rhs_lanes<TL, NRP>())
-      node_product_mr<T, ND, NRP, D16>(m, val, u, n, cur, lane, am);
+    T wg = T(0), outv[KE];
+    if constexpr (RG)
+      wg = node_product_rg<T, ND, NRP, D16>(m, val, u, n, cur, lane);
+    else if constexpr (QUADS)
+      node_product_quads<ND, TL, NRP, D16>(m, val, u, n, cur, lane, outv);
     else if constexpr (lds_reduce<T, TL, NRP>())
       node_product_lds<T, ND, TL, NRP, D16>(m, val, u, n, cur, lane, team, outv);
     else
       node_product_at<T, ND, TL, NRP, D16>(m, val, u, n, cur, lane, acc);
 #pragma unroll
     for (int k = 0; k < KE; ++k) {
-      const int e = lane + k * TL;
+      const int e = e0 + k * TL;
       if (lv && e < NE) {
         T w = T(0);
-        if constexpr (rhs_lanes<TL, NRP>()) {
-          w = pick_entry<T, ND, NRP>(am, e);  // e = lane: rhs lane % NRP
-        } else if constexpr (lds_reduce<T, TL, NRP>()) {
+        if constexpr (RG) {
+          w = wg;
+        } else if constexpr (QUADS || lds_reduce<T, TL, NRP>()) {
           w = outv[k];
         } else {
 #pragma unroll
@@ -641,6 +797,11 @@ __device__ __forceinline__ void spmv_dir_body(const tfm_mesh_t &m, const T *__re
         dot += (double)pv * (double)sv;
       }
     }
+  }
+  // the partial sums take thread t's value for rhs t % NRP
+  if constexpr (RG || QUADS) {
+    const int l = threadIdx.x % 64;
+    dot = __shfl(dot, l / NRP * NRP + rg_lane<NRP>(l % NRP), 64);
   }
   double v[1] = {dot};
   write_block_partials<1, NRP>(v, sh, st.part_pq);
