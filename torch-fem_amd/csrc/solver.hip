@@ -1366,11 +1366,10 @@ static SpmvShape spmv_shape(const tfm_mesh_t &m, int nrp) {
 
 // Team width TL: 4 (FP64 scalar fields with short rows), 8 (rows of at most
 // 16 neighbour blocks on average), 16 or 32 lanes per node, or a whole wave
-// with the rhs
-// across lanes (node_product_mr) for FP64 with four or more right-hand sides,
-// where a lane cannot hold ND*NRP doubles without losing occupancy. (In FP32
-// the lane-per-block product measured faster for 16 rhs: 274 against 307 us
-// on Hexa2 32^3.) T and NRP must be in scope.
+// with the rhs across lanes (node_product_rg) for FP64 with four or more
+// right-hand sides, where a lane cannot hold ND*NRP doubles without losing
+// occupancy. (In FP32 a wave per node took 55 us for 16 rhs on Hexa2 21x19x23,
+// 32 lanes per node 44: node_product_quads.) T and NRP must be in scope.
 #define TFM_WIDE_TEAM (sizeof(T) == 8 && NRP >= 4)
 #define TFM_TEAM_SWITCH(tl, ...)                                                               \
   switch (TFM_WIDE_TEAM ? 64 : (tl)) {                                                         \
