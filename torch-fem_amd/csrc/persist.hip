@@ -30,8 +30,13 @@
 // decisions; results do not vary from run to run.
 //
 // Every wait is bounded (50 ms): if some block has not been scheduled by then
-// (another process holds CUs), all blocks leave, x is still a valid guess,
-// and the caller solves on the general path, with this handle from then on.
+// (another process holds CUs), it sets the abort word and leaves, and with it
+// every block that waits for it. x is still a valid guess, some blocks having
+// folded a correction into it and others not, and the caller solves on the
+// general path, with this handle from then on. Whether a solve counts is decided
+// by the abort word, read once the kernel has ended, not by block 0: at the
+// last exchange of a solve block 0 may have seen every block that another gave
+// up on, and at b = 0 the block that left has not cleared its part of x.
 //
 // Of the 6.4 us of an iteration on a 14^3 Hexa1 cube (84 blocks) about 2.6 are
 // the wait for eta, 0.7 and 0.8 those for the neighbours' u and for (r.u, r.r),
@@ -66,10 +71,10 @@ struct PersistArgs {
   double *x;
   void *ug, *pg;
   unsigned long long *slots;
-  unsigned long long *abort;
   PersistResult *res;
   double rtol, delta, final_rtol;
   int max_iter, extended;
+  unsigned quit;  // the exchange whose wait the last block gives up at once (0: none)
 };
 
 template <typename T> __device__ __forceinline__ T dev_load(const T *p) {
@@ -143,6 +148,11 @@ __device__ __forceinline__ void publish(double (&v)[NV], Exchange &X, unsigned e
 template <int N>
 __device__ __forceinline__ bool poll(const unsigned long long *at, unsigned epoch,
                                      unsigned long long (&w)[N], const PersistArgs &A) {
+  unsigned long long *abort = &A.res->abort;
+  if (epoch == A.quit && blockIdx.x == gridDim.x - 1) {
+    dev_store(abort, 1ull);
+    return false;
+  }
   const long long t0 = wall_clock64();
   for (int spin = 0;; ++spin) {
     bool ok = true;
@@ -151,8 +161,8 @@ __device__ __forceinline__ bool poll(const unsigned long long *at, unsigned epoc
 #pragma unroll
     for (int k = 0; k < N; ++k) ok &= (unsigned)(w[k] >> 32) == epoch;
     if (ok) return true;
-    if (spin % 32 == 31 && (dev_load(A.abort) != 0 || wall_clock64() - t0 > P_WAIT_TICKS)) {
-      dev_store(A.abort, 1ull);
+    if (spin % 32 == 31 && (dev_load(abort) != 0 || wall_clock64() - t0 > P_WAIT_TICKS)) {
+      dev_store(abort, 1ull);
       return false;
     }
   }
@@ -808,15 +818,15 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
   A.ug = J.u;
   A.pg = J.p;
   A.slots = slots;
-  A.abort = slots + PERSIST_SLOTS;
-  A.res = reinterpret_cast<PersistResult *>(slots + PERSIST_SLOTS + 8);
+  A.res = reinterpret_cast<PersistResult *>(slots + PERSIST_SLOTS);
   A.rtol = J.rtol;
   A.delta = J.delta;
   A.final_rtol = J.final_rtol;
   A.max_iter = J.max_iter;
   A.extended = J.extended;
-  hipLaunchKernelGGL(k_clear_slots, dim3((PERSIST_SLOTS + 8 + 255) / 256), dim3(256), 0, s, slots,
-                     PERSIST_SLOTS + 8);
+  A.quit = (unsigned)env_int("TFM_PCG_PERSIST_QUIT", 0);
+  constexpr int words = PERSIST_SCRATCH_BYTES / sizeof(unsigned long long);
+  hipLaunchKernelGGL(k_clear_slots, dim3((words + 255) / 256), dim3(256), 0, s, slots, words);
   TFM_CHECK_LAUNCH();
   int rc = TFM_OK;
   if (csr) rc = launch<double, 1, 8, true>(s, grid, A);
@@ -832,6 +842,7 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
   TFM_CHECK_HIP(hipMemcpyAsync(J.h_res, A.res, sizeof(PersistResult), hipMemcpyDeviceToHost, s));
   TFM_CHECK_HIP(hipStreamSynchronize(s));
   *res = *J.h_res;
+  if (res->abort) res->status = PERSIST_ABORTED;
   *ran = res->status != PERSIST_NOFIT && res->status != PERSIST_ABORTED;
   return TFM_OK;
 }

@@ -131,7 +131,9 @@ enum {
   PERSIST_ABORTED = 6 // a block did not arrive in time: x holds a valid guess
 };
 
+// abort is set by any block that gives up a wait, the others by block 0.
 struct PersistResult {
+  unsigned long long abort;
   int status, iters, segments, pad;
   double relres;
 };
@@ -140,9 +142,9 @@ constexpr int PERSIST_MAX_BLOCKS = 256;
 constexpr int PERSIST_COPIES = 8;
 // exchange slots: [parity][copy][value][2 words][block]
 constexpr int PERSIST_SLOTS = 2 * PERSIST_COPIES * 3 * 2 * PERSIST_MAX_BLOCKS;
-// device scratch of one solve: the slots, an abort word and the result
+// device scratch of one solve: the slots and the result
 constexpr size_t PERSIST_SCRATCH_BYTES =
-    sizeof(unsigned long long) * (PERSIST_SLOTS + 8) + sizeof(PersistResult);
+    sizeof(unsigned long long) * PERSIST_SLOTS + sizeof(PersistResult);
 
 struct PersistJob {
   // rows: the node blocks of a mesh, or a general CSR matrix (m == nullptr)
