@@ -341,6 +341,17 @@ int tfm_pcg_timing(tfm_pcg_t *h, int32_t enable, double *spmv_ms,
  * reference, which solves in FP64 only. */
 int tfm_pcg_fp64_fallback(const tfm_pcg_t *h, int32_t *fp64_iters);
 
+/* How the last solve of the handle ran (the FP64 part, if it ended in one):
+ * in the persistent kernel of small systems, or on the general path, and then
+ * whether the kernel was tried first. No counterpart in the reference. */
+enum {
+  TFM_PATH_GENERAL = 0,    /* general path */
+  TFM_PATH_PERSISTENT = 1, /* the whole solve in one kernel */
+  TFM_PATH_NO_FIT = 2,     /* general, the kernel's index sets did not fit LDS */
+  TFM_PATH_GAVE_UP = 3     /* general, a block of the kernel did not get a CU in time */
+};
+int tfm_pcg_path(const tfm_pcg_t *h, int32_t *path);
+
 /* ------------------------------------------- two-level preconditioner */
 /* Coarse space of TFM_PC_TWO_LEVEL, in the place of the aggregation AMG the
  * reference reaches through AmgX (sparse.py:422-442, amgx.py:71-98): nodes

@@ -2087,6 +2087,7 @@ struct tfm_pcg {
   void *persist = nullptr;                                 // scratch of the persistent solver
   PersistResult *h_persist = nullptr;                      // its outcome (pinned)
   bool persist_off = false;  // a persistent solve found the GPU shared (PERSIST_ABORTED)
+  int path = TFM_PATH_GENERAL;  // of the last solve
   // optional event timing of the SpMV launches (kernel A) of the iterations
   // the FP32 arithmetic of the last mixed solve broke down (p.Kp <= 0, or a
   // true residual that stopped falling), and the FP64 iterations that finished it
@@ -2334,6 +2335,12 @@ extern "C" int tfm_spd_inverse(tfm_stream_t stream, int32_t n, double *a, double
 extern "C" int tfm_pcg_fp64_fallback(const tfm_pcg_t *h, int32_t *fp64_iters) {
   TFM_REQUIRE(h != nullptr && fp64_iters != nullptr, "null argument");
   *fp64_iters = h->fallback_iters;
+  return TFM_OK;
+}
+
+extern "C" int tfm_pcg_path(const tfm_pcg_t *h, int32_t *path) {
+  TFM_REQUIRE(h != nullptr && path != nullptr, "null argument");
+  *path = h->path;
   return TFM_OK;
 }
 
@@ -2751,6 +2758,7 @@ int run_pcg(tfm_pcg *h, hipStream_t s, int64_t n_nod, Ops<T> &ops, const double 
 // the general path, whose launches they time.
 bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, double *relres,
                  int32_t *outer, int *rc) {
+  h->path = TFM_PATH_GENERAL;
   if (h->timing || h->persist_off) return false;
   job.u = h->u;
   job.p = h->p;
@@ -2763,8 +2771,11 @@ bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, dou
   if (*rc != TFM_OK) return true;
   if (!ran) {
     h->persist_off = res.status == PERSIST_ABORTED;
+    if (res.status == PERSIST_ABORTED) h->path = TFM_PATH_GAVE_UP;
+    if (res.status == PERSIST_NOFIT) h->path = TFM_PATH_NO_FIT;
     return false;
   }
+  h->path = TFM_PATH_PERSISTENT;
   iters[0] = res.iters;
   relres[0] = res.relres;
   if (outer) *outer = res.segments;
@@ -2874,6 +2885,7 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
     return fem_residual(h, s, *sys, bb, xx, res, rr, b2, extended);
   };
   h->fallback_iters = 0;
+  h->path = TFM_PATH_GENERAL;
   TFM_ND_SWITCH(m.ndof, TFM_NRP_SWITCH(nrp, {
     auto small = [&](bool fp64, int32_t *its, int32_t *out, int *rcs) -> bool {
       if (NRP != 1 || cs || !sys->val64) return false;

@@ -30,6 +30,7 @@ MAT_ISO, MAT_GENERAL, MAT_HEAT_ISO, MAT_HEAT_GENERAL = 1, 2, 3, 4
 PREC_FP64, PREC_MIXED = 0, 1
 PC_JACOBI, PC_BLOCK_JACOBI, PC_TWO_LEVEL = 0, 1, 2
 FP32_PLAIN, FP32_DIFF = 0, 1
+PCG_PATH = ("general", "persistent", "no_fit", "gave_up")  # TFM_PATH_*
 
 P = C.c_void_p
 I32 = C.c_int32
@@ -149,6 +150,7 @@ _SIGNATURES: dict[str, tuple[list[Any], Any]] = {
     ),
     "tfm_pcg_timing": ([P, I32, C.POINTER(F64), C.POINTER(I64)], C.c_int),
     "tfm_pcg_fp64_fallback": ([P, C.POINTER(I32)], C.c_int),
+    "tfm_pcg_path": ([P, C.POINTER(I32)], C.c_int),
     "tfm_coarse_create": ([C.POINTER(P), P, I32, P, P, P, P, P, P, I64, P, P], C.c_int),
     "tfm_coarse_destroy": ([P], C.c_int),
     "tfm_coarse_size": ([P, C.POINTER(I32)], C.c_int),

@@ -151,6 +151,13 @@ class PCGSolver:
             self.nrhs = nrhs
             self._create()
 
+    @property
+    def path(self) -> str:
+        """How the last solve ran (L.PCG_PATH, tfm_pcg_path)."""
+        p = L.I32()
+        L.check(L.lib().tfm_pcg_path(self._h, C.byref(p)))
+        return L.PCG_PATH[p.value]
+
     def timing(self, stride: int) -> tuple[float, int]:
         """Event-timed inner SpMV launches since the last call (ms, count);
         resets the totals, then times the SpMV of every `stride`-th
@@ -185,7 +192,7 @@ class PCGSolver:
         L.check(L.lib().tfm_pcg_fp64_fallback(self._h, C.byref(fb)))
         info = dict(iterations=list(its), relres=list(rel), outer=int(outer.value),
                     time=time.perf_counter() - t0, precision=precision, preconditioner=preconditioner,
-                    fp64_fallback=int(fb.value))
+                    fp64_fallback=int(fb.value), path=self.path)
         if rc == L.TFM_ERR_NOCONV:
             msg = L.lib().tfm_last_error().decode(errors="replace")
             raise RuntimeError(f"PCG did not converge ({msg}): {info}")
@@ -199,7 +206,7 @@ class PCGSolver:
         rc = L.lib().tfm_csr_pcg_solve(self._h, L.stream_of(self.device), self.n, L.ptr(rowptr),
                                        L.ptr(col), L.ptr(val), L.ptr(b), L.ptr(x), float(rtol),
                                        C.byref(its), C.byref(rel))
-        info = dict(iterations=int(its.value), relres=float(rel.value))
+        info = dict(iterations=int(its.value), relres=float(rel.value), path=self.path)
         if rc == L.TFM_ERR_NOCONV:
             msg = L.lib().tfm_last_error().decode(errors="replace")
             raise RuntimeError(f"CG failed after {info['iterations']} iterations: {msg}")
