@@ -52,5 +52,5 @@ def test_csr_rows(n, path):
 
 
 def test_a_wait_given_up_is_reported(monkeypatch):
-    monkeypatch.setenv("TFM_PCG_PERSIST_QUIT", "5")
+    monkeypatch.setenv("TFM_PCG_PERSIST_QUIT", "2")
     assert fem_path(model_of("hexa1", (6, 6, 6)), stol=1e-9) == "gave_up"

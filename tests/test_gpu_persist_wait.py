@@ -1,7 +1,8 @@
 """A wait of the persistent small-system solver (csrc/persist.hip) that is given
-up: TFM_PCG_PERSIST_QUIT makes the last block give up the wait for one exchange,
-as it would after 50 ms without the others; every block then leaves and the
-general path finishes the solve from whatever x the blocks have left.
+up: TFM_PCG_PERSIST_QUIT makes the last block leave at one point of the solve, as
+it would after 50 ms without the others: 2 k - 1 where it waits for the k-th
+residual, 2 k before it folds its k-th correction into x. Every block then leaves
+and the general path finishes the solve from whatever x the blocks have left.
 
 Tolerance of a solution: as in test_gpu_persist.py, cond(K) (stol + 1e-14).
 """
@@ -19,7 +20,7 @@ DT = torch.float64
 @pytest.mark.parametrize("quit_at", [1, 2])
 def test_zero_load_from_a_warm_start(quit_at, monkeypatch):
     """b = 0 gives x = 0 whatever the guess, also where the last block leaves
-    before it has cleared its part (exchange 2 is the one that finds b = 0)."""
+    before it has cleared its part (the first residual tells that b = 0)."""
     A, b = grid_matrix(3000)
     rowptr, col, val = _csr_arrays(A, b.device)
     monkeypatch.setenv("TFM_PCG_PERSIST_QUIT", str(quit_at))
@@ -33,13 +34,13 @@ def test_zero_load_from_a_warm_start(quit_at, monkeypatch):
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("kind,n", [("hexa1", (6, 6, 6)), ("quad1", (37, 23))])
 def test_solution_after_a_wait_given_up(kind, n, precision, monkeypatch):
-    """Every exchange of the first segment, and some of the later ones, where x
-    holds the corrections of some blocks only; from zero and from a warm start."""
+    """Before and within the folds, where x holds the correction of some blocks
+    only; from zero and from a warm start."""
     m = model_of(kind, n)
     f = m._neumann
     m.solve()
     _, x, cond = dense(m)
-    for quit_at in (*range(1, 11), 25, 40, 41, 42, 43, 60, 61):
+    for quit_at in range(1, 9):
         m = model_of(kind, n)  # its own solver handle
         monkeypatch.setenv("TFM_PCG_PERSIST_QUIT", str(quit_at))
         for stol, scale in ((1e-9, 1.0), (1e-12, 1.5)):

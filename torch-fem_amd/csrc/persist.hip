@@ -74,7 +74,7 @@ struct PersistArgs {
   PersistResult *res;
   double rtol, delta, final_rtol;
   int max_iter, extended;
-  unsigned quit;  // the exchange whose wait the last block gives up at once (0: none)
+  int quit;  // the point where the last block gives up (0: none), see `quits`
 };
 
 template <typename T> __device__ __forceinline__ T dev_load(const T *p) {
@@ -149,10 +149,6 @@ template <int N>
 __device__ __forceinline__ bool poll(const unsigned long long *at, unsigned epoch,
                                      unsigned long long (&w)[N], const PersistArgs &A) {
   unsigned long long *abort = &A.res->abort;
-  if (epoch == A.quit && blockIdx.x == gridDim.x - 1) {
-    dev_store(abort, 1ull);
-    return false;
-  }
   const long long t0 = wall_clock64();
   for (int spin = 0;; ++spin) {
     bool ok = true;
@@ -223,7 +219,9 @@ __device__ __forceinline__ bool exchange(double (&v)[NV], Exchange &X, unsigned 
   return collect<NV>(v, X, epoch, A);
 }
 
-template <typename T, int ND, int TL, bool CSR>
+// QUIT: the last block gives up at point A.quit. (With that test in the kernels of
+// QUIT = false too, an iteration of three DOFs took 2% longer.)
+template <typename T, int ND, int TL, bool CSR, bool QUIT = false>
 __global__ void __launch_bounds__(PT) k_pcg_persist(PersistArgs A) {
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ Exchange X;
@@ -542,6 +540,15 @@ __global__ void __launch_bounds__(PT) k_pcg_persist(PersistArgs A) {
     }
   };
 
+  // A wait given up on request, as after P_WAIT_TICKS: the last block's for the
+  // k-th residual (point 2 k - 1), or the one before it folds its k-th correction
+  // into x (point 2 k).
+  auto quits = [&](int point) -> bool {
+    if (!QUIT || point != A.quit || blockIdx.x != gridDim.x - 1) return false;
+    if (tid == 0) dev_store(&A.res->abort, 1ull);
+    return true;
+  };
+
   // ------------------------------------------------------------- the solve
   double bnorm = 0.0, rnow = 0.0, rprev = 0.0;
   double g = 0.0, den = 0.0;  // r.u of this iteration and of the last one run
@@ -553,7 +560,8 @@ __global__ void __launch_bounds__(PT) k_pcg_persist(PersistArgs A) {
     double v2[2] = {0.0, 0.0};
     if (FP64 && resident) residual(reinterpret_cast<const double *>(lval), v2);
     else residual(A.val64 + v_beg, v2);
-    if (!exchange<2>(v2, X, epoch, A)) {
+    publish<2>(v2, X, ++epoch, A);
+    if (quits(2 * nseg + 1) || !collect<2>(v2, X, epoch, A)) {
       status = PERSIST_ABORTED;
       break;
     }
@@ -706,6 +714,10 @@ __global__ void __launch_bounds__(PT) k_pcg_persist(PersistArgs A) {
       status = PERSIST_MAXITER;
       break;
     }
+    if (quits(2 * nseg + 2)) {
+      status = PERSIST_ABORTED;
+      break;
+    }
     // fold the correction into x
     ++nseg;
     for (int i = tid; i < nloc * ND; i += PT) {
@@ -726,17 +738,18 @@ __global__ void k_clear_slots(unsigned long long *slots, int n) {
   if (i < n) slots[i] = 0ull;
 }
 
-template <typename T, int ND, int TL, bool CSR>
+template <typename T, int ND, int TL, bool CSR, bool QUIT = false>
 int launch(hipStream_t s, unsigned grid, const PersistArgs &A) {
-  const void *fn = reinterpret_cast<const void *>(&k_pcg_persist<T, ND, TL, CSR>);
+  const void *fn = reinterpret_cast<const void *>(&k_pcg_persist<T, ND, TL, CSR, QUIT>);
   TFM_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P_LDS));
-  hipLaunchKernelGGL((k_pcg_persist<T, ND, TL, CSR>), dim3(grid), dim3(PT), P_LDS, s, A);
+  hipLaunchKernelGGL((k_pcg_persist<T, ND, TL, CSR, QUIT>), dim3(grid), dim3(PT), P_LDS, s, A);
   TFM_CHECK_LAUNCH();
   return TFM_OK;
 }
 
 template <typename T, int ND>
 int launch_team(hipStream_t s, unsigned grid, double deg, const PersistArgs &A) {
+  if (A.quit > 0) return launch<T, ND, 8, false, true>(s, grid, A);
   if (deg > 32.0) return launch<T, ND, 32, false>(s, grid, A);
   if (deg > 16.0) return launch<T, ND, 16, false>(s, grid, A);
   return launch<T, ND, 8, false>(s, grid, A);
@@ -824,12 +837,13 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
   A.final_rtol = J.final_rtol;
   A.max_iter = J.max_iter;
   A.extended = J.extended;
-  A.quit = (unsigned)env_int("TFM_PCG_PERSIST_QUIT", 0);
+  A.quit = env_int("TFM_PCG_PERSIST_QUIT", 0);
   constexpr int words = PERSIST_SCRATCH_BYTES / sizeof(unsigned long long);
   hipLaunchKernelGGL(k_clear_slots, dim3((words + 255) / 256), dim3(256), 0, s, slots, words);
   TFM_CHECK_LAUNCH();
   int rc = TFM_OK;
-  if (csr) rc = launch<double, 1, 8, true>(s, grid, A);
+  if (csr && A.quit > 0) rc = launch<double, 1, 8, true, true>(s, grid, A);
+  else if (csr) rc = launch<double, 1, 8, true>(s, grid, A);
   else if (J.fp64)
     rc = nd == 1   ? launch_team<double, 1>(s, grid, deg, A)
          : nd == 2 ? launch_team<double, 2>(s, grid, deg, A)
