@@ -27,7 +27,8 @@
 //     sees the u. No fence is needed, and none is paid for: an agent-scope
 //     fence per block measured 6 to 16 us on 128 to 256 blocks.
 // All blocks form the same sums in the same order, so they take the same
-// decisions; results do not vary from run to run.
+// decisions; results do not vary from run to run, unless a wait is given up (see
+// below).
 //
 // Every wait is bounded (50 ms): if some block has not been scheduled by then
 // (another process holds CUs), it sets the abort word and leaves, and with it
@@ -45,8 +46,8 @@
 #include "solver_common.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
+#include <mutex>
 #include <type_traits>
 
 namespace tfm {
@@ -756,15 +757,10 @@ int launch_team(hipStream_t s, unsigned grid, double deg, const PersistArgs &A) 
 }
 
 // One persistent solve per device at a time in this process: two of them on
-// different streams could each hold part of the CUs and wait for the rest.
-std::atomic<int> g_busy[64];
-
-struct BusyGuard {
-  std::atomic<int> *flag = nullptr;
-  ~BusyGuard() {
-    if (flag) flag->store(0, std::memory_order_release);
-  }
-};
+// different streams could each hold part of the CUs and wait for the rest. A
+// solve waits its turn rather than taking the general path, whose sums have
+// another order: its results then do not depend on what other threads do.
+std::mutex g_turn[64];
 
 }  // namespace
 
@@ -806,11 +802,6 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
                          : nd == 2 ? (J.fp64 ? fixed_lds<double, 2>(npb) : fixed_lds<float, 2>(npb))
                                    : (J.fp64 ? fixed_lds<double, 3>(npb) : fixed_lds<float, 3>(npb));
   if (fixed > P_LDS / 2) return TFM_OK;
-  int expected = 0;
-  if (!g_busy[dev].compare_exchange_strong(expected, 1, std::memory_order_acquire)) return TFM_OK;
-  BusyGuard guard;
-  guard.flag = &g_busy[dev];
-
   auto *slots = reinterpret_cast<unsigned long long *>(J.scratch);
   PersistArgs A{};
   A.n_nod = n_nod;
@@ -841,6 +832,10 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
   constexpr int words = PERSIST_SCRATCH_BYTES / sizeof(unsigned long long);
   hipLaunchKernelGGL(k_clear_slots, dim3((words + 255) / 256), dim3(256), 0, s, slots, words);
   TFM_CHECK_LAUNCH();
+  // what the stream still holds is awaited before the turn, not within it: a
+  // turn then lasts as long as its kernel, which waits for nobody else's work
+  TFM_CHECK_HIP(hipStreamSynchronize(s));
+  std::lock_guard<std::mutex> turn(g_turn[dev]);
   int rc = TFM_OK;
   if (csr && A.quit > 0) rc = launch<double, 1, 8, true, true>(s, grid, A);
   else if (csr) rc = launch<double, 1, 8, true>(s, grid, A);
