@@ -53,4 +53,5 @@ def test_csr_rows(n, path):
 
 def test_a_wait_given_up_is_reported(monkeypatch):
     monkeypatch.setenv("TFM_PCG_PERSIST_QUIT", "2")
+    monkeypatch.setenv("TFM_PCG_PERSIST_REST_MS", "0")
     assert fem_path(model_of("hexa1", (6, 6, 6)), stol=1e-9) == "gave_up"

@@ -7,6 +7,9 @@ and the general path finishes the solve from whatever x the blocks have left.
 Tolerance of a solution: as in test_gpu_persist.py, cond(K) (stol + 1e-14).
 """
 
+import threading
+import time
+
 import pytest
 import torch
 
@@ -15,6 +18,12 @@ from torchfem.sparse import PCGSolver, _csr_arrays
 
 pytestmark = pytest.mark.gpu
 DT = torch.float64
+
+
+@pytest.fixture(autouse=True)
+def no_rest(monkeypatch):
+    """The solves after one that gave up take the persistent kernel again."""
+    monkeypatch.setenv("TFM_PCG_PERSIST_REST_MS", "0")
 
 
 @pytest.mark.parametrize("quit_at", [1, 2])
@@ -48,3 +57,32 @@ def test_solution_after_a_wait_given_up(kind, n, precision, monkeypatch):
             u = m.solve(precision=precision, preconditioner="block_jacobi", stol=stol,
                         use_cached_solve=True)[0].reshape(-1) / scale
             assert float((u - x).norm() / x.norm()) <= cond * (stol + 1e-14), quit_at
+
+
+def test_rest_after_a_wait_given_up(monkeypatch):
+    """The next solves of the thread do not wait again, whatever their handle;
+    other threads' do as before, and so does the thread's after the rest."""
+    A, b = grid_matrix(3000)
+    rowptr, col, val = _csr_arrays(A, b.device)
+
+    def path(out):
+        solver = PCGSolver(3000, 1, b.device)  # as sparse_solve: a handle per solve
+        out.append(solver.solve_csr(rowptr, col, val, b, torch.zeros_like(b), 1e-10)["path"])
+        solver.close()
+        return out[-1]
+
+    assert path([]) == "persistent"
+    monkeypatch.setenv("TFM_PCG_PERSIST_REST_MS", "2000")
+    monkeypatch.setenv("TFM_PCG_PERSIST_QUIT", "2")
+    t0 = time.monotonic()
+    assert path([]) == "gave_up"
+    monkeypatch.setenv("TFM_PCG_PERSIST_QUIT", "0")
+    seen = path([])
+    other = []
+    thread = threading.Thread(target=path, args=(other,))
+    thread.start()
+    thread.join()
+    assert time.monotonic() - t0 < 1.9  # all of this within the rest
+    assert seen == "general" and other == ["persistent"]
+    time.sleep(2.1)
+    assert path([]) == "persistent"

@@ -34,7 +34,8 @@
 // (another process holds CUs), it sets the abort word and leaves, and with it
 // every block that waits for it. x is still a valid guess, some blocks having
 // folded a correction into it and others not, and the caller solves on the
-// general path, with this handle from then on. Whether a solve counts is decided
+// general path, as do the thread's solves on the device for the next 4 s (another
+// process on the GPU tends to stay; a solver handle may live for one solve). Whether a solve counts is decided
 // by the abort word, read once the kernel has ended, not by block 0: at the
 // last exchange of a solve block 0 may have seen every block that another gave
 // up on, and at b = 0 the block that left has not cleared its part of x.
@@ -46,6 +47,7 @@
 #include "solver_common.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -762,6 +764,10 @@ int launch_team(hipStream_t s, unsigned grid, double deg, const PersistArgs &A) 
 // another order: its results then do not depend on what other threads do.
 std::mutex g_turn[64];
 
+// Until when the calling thread's solves on a device take the general path,
+// because one of them has given up a wait.
+thread_local std::chrono::steady_clock::time_point g_rest[64];
+
 }  // namespace
 
 int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *ran) {
@@ -776,6 +782,7 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
   TFM_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   TFM_CHECK_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
   if (dev >= 64 || lds < 160 * 1024) return TFM_OK;
+  if (std::chrono::steady_clock::now() < g_rest[dev]) return TFM_OK;
   const int max_blocks = std::min(cus, PERSIST_MAX_BLOCKS);
   const unsigned size = J.fp64 ? 8u : 4u;
   const double nnz = csr ? 7.0 * n_nod : (double)J.m->nnz;
@@ -851,7 +858,11 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
   TFM_CHECK_HIP(hipMemcpyAsync(J.h_res, A.res, sizeof(PersistResult), hipMemcpyDeviceToHost, s));
   TFM_CHECK_HIP(hipStreamSynchronize(s));
   *res = *J.h_res;
-  if (res->abort) res->status = PERSIST_ABORTED;
+  if (res->abort) {
+    res->status = PERSIST_ABORTED;
+    g_rest[dev] = std::chrono::steady_clock::now() +
+                  std::chrono::milliseconds(env_int("TFM_PCG_PERSIST_REST_MS", 4000));
+  }
   *ran = res->status != PERSIST_NOFIT && res->status != PERSIST_ABORTED;
   return TFM_OK;
 }

@@ -2086,7 +2086,6 @@ struct tfm_pcg {
   double *h_scal = nullptr;                                // a batch's scalars
   void *persist = nullptr;                                 // scratch of the persistent solver
   PersistResult *h_persist = nullptr;                      // its outcome (pinned)
-  bool persist_off = false;  // a persistent solve found the GPU shared (PERSIST_ABORTED)
   int path = TFM_PATH_GENERAL;  // of the last solve
   // optional event timing of the SpMV launches (kernel A) of the iterations
   // the FP32 arithmetic of the last mixed solve broke down (p.Kp <= 0, or a
@@ -2759,7 +2758,7 @@ int run_pcg(tfm_pcg *h, hipStream_t s, int64_t n_nod, Ops<T> &ops, const double 
 bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, double *relres,
                  int32_t *outer, int *rc) {
   h->path = TFM_PATH_GENERAL;
-  if (h->timing || h->persist_off) return false;
+  if (h->timing) return false;
   job.u = h->u;
   job.p = h->p;
   job.scratch = h->persist;
@@ -2770,7 +2769,6 @@ bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, dou
   *rc = persist_solve(s, job, &res, &ran);
   if (*rc != TFM_OK) return true;
   if (!ran) {
-    h->persist_off = res.status == PERSIST_ABORTED;
     if (res.status == PERSIST_ABORTED) h->path = TFM_PATH_GAVE_UP;
     if (res.status == PERSIST_NOFIT) h->path = TFM_PATH_NO_FIT;
     return false;
