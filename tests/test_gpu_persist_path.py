@@ -6,6 +6,10 @@ import pytest
 import torch
 
 from test_gpu_persist import CASES, DT, grid_matrix, model_of
+from torchfem import Solid
+from torchfem.elements import linear_to_quadratic
+from torchfem.materials import IsotropicElasticity3D
+from torchfem.mesh import cube_hexa
 from torchfem.sparse import PCGSolver, _csr_arrays
 
 pytestmark = pytest.mark.gpu
@@ -49,6 +53,26 @@ def test_csr_rows(n, path):
     solver = PCGSolver(n, 1, b.device)
     assert solver.solve_csr(rowptr, col, val, b, torch.zeros_like(b), 1e-10)["path"] == path
     solver.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_a_mesh_that_does_not_fit_is_tried_once(precision):
+    """Hexa2 with its nodes numbered at random: too many distinct neighbours for
+    a block's LDS. The model's next solves do not try again."""
+    nodes, el = linear_to_quadratic(*cube_hexa(19, 19, 19))
+    p = torch.randperm(len(nodes), generator=torch.Generator().manual_seed(0))
+    inv = torch.empty_like(p)
+    inv[p] = torch.arange(len(p))
+    m = Solid(nodes.to(DT)[p].cuda(), inv[el].cuda(),
+              IsotropicElasticity3D(torch.tensor(1000.0, dtype=DT, device="cuda"),
+                                    torch.tensor(0.3, dtype=DT, device="cuda")))
+    m.constraints[m.nodes[:, 0] == 0.0] = True
+    m.forces[m.nodes[:, 0] == 1.0, 1] = 1.0
+    paths = []
+    for _ in range(2):  # one or more linear solves each
+        m.solve(precision=precision, preconditioner="block_jacobi", stol=1e-6)
+        paths += [p["path"] for p in m.last_solve_info["forward"]["pcg"]]
+    assert paths == ["no_fit"] + ["general"] * (len(paths) - 1)
 
 
 def test_a_wait_given_up_is_reported(monkeypatch):

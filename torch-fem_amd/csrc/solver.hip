@@ -2087,6 +2087,10 @@ struct tfm_pcg {
   void *persist = nullptr;                                 // scratch of the persistent solver
   PersistResult *h_persist = nullptr;                      // its outcome (pinned)
   int path = TFM_PATH_GENERAL;  // of the last solve
+  // non-zeros of the mesh system that last did not fit the persistent solver, in
+  // FP32 and in FP64 (a model's systems share a pattern: the launch and the round
+  // trip that find this out, 30 to 80 us, are not paid for at every solve)
+  int64_t no_fit[2] = {-1, -1};
   // optional event timing of the SpMV launches (kernel A) of the iterations
   // the FP32 arithmetic of the last mixed solve broke down (p.Kp <= 0, or a
   // true residual that stopped falling), and the FP64 iterations that finished it
@@ -2758,7 +2762,7 @@ int run_pcg(tfm_pcg *h, hipStream_t s, int64_t n_nod, Ops<T> &ops, const double 
 bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, double *relres,
                  int32_t *outer, int *rc) {
   h->path = TFM_PATH_GENERAL;
-  if (h->timing) return false;
+  if (h->timing || (job.m && job.m->nnz == h->no_fit[job.fp64])) return false;
   job.u = h->u;
   job.p = h->p;
   job.scratch = h->persist;
@@ -2770,7 +2774,10 @@ bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, dou
   if (*rc != TFM_OK) return true;
   if (!ran) {
     if (res.status == PERSIST_ABORTED) h->path = TFM_PATH_GAVE_UP;
-    if (res.status == PERSIST_NOFIT) h->path = TFM_PATH_NO_FIT;
+    if (res.status == PERSIST_NOFIT) {
+      h->path = TFM_PATH_NO_FIT;
+      if (job.m) h->no_fit[job.fp64] = job.m->nnz;
+    }
     return false;
   }
   h->path = TFM_PATH_PERSISTENT;
