@@ -2070,7 +2070,7 @@ struct tfm_pcg {
   double *x = nullptr, *r = nullptr, *u = nullptr, *p = nullptr, *s = nullptr;
   double *minv = nullptr;                                  // sized n*3 doubles
   double *xm = nullptr, *r64 = nullptr, *f64 = nullptr;    // FP64 work vectors [n]
-  double *xy64 = nullptr;                                  // [2][n][nrp], several rhs (cols)
+  double *xy64 = nullptr;                                  // [2][n][nrp], see joint_buffers
   double *part_cols = nullptr;                             // [RBV][2][nrp]
   double *work = nullptr;                                  // internal-force scratch
   int64_t work_len = 0;
@@ -2130,10 +2130,7 @@ static int pcg_alloc(tfm_pcg *h) {
   TFM_CHECK_HIP(hipMalloc(&h->part_res, sizeof(double) * (size_t)h->res_cap * 2));
   TFM_CHECK_HIP(hipMalloc(&h->coef, sizeof(PcgCoef) * 2));
   TFM_CHECK_HIP(hipMalloc(&h->res2, sizeof(double) * 2 * MAXR));
-  if (nrp > 1) {
-    TFM_CHECK_HIP(hipMalloc(&h->xy64, 2 * vbytes));
-    TFM_CHECK_HIP(hipMalloc(&h->part_cols, sizeof(double) * RBV * 2 * nrp));
-  }
+  if (nrp > 1) TFM_CHECK_HIP(hipMalloc(&h->part_cols, sizeof(double) * RBV * 2 * nrp));
   TFM_CHECK_HIP(hipMalloc(&h->done, sizeof(int) * nrp));
   TFM_CHECK_HIP(hipMalloc(&h->alldone, sizeof(int)));
   TFM_CHECK_HIP(hipMalloc(&h->segf, sizeof(int) * nrp));
@@ -2145,6 +2142,20 @@ static int pcg_alloc(tfm_pcg *h) {
   TFM_CHECK_HIP(hipHostMalloc(&h->h_persist, sizeof(PersistResult), hipHostMallocDefault));
   for (auto &e : h->ev) TFM_CHECK_HIP(hipEventCreate(&e));
   return TFM_OK;
+}
+
+// The two vectors of the joint refinement of several right-hand sides, from the
+// first solve that uses it: they are two fifths of what the Krylov vectors take,
+// and tolerances below 1e-10 or systems without FP64 values do without. False if
+// there is no memory for them (or TFM_PCG_JOINT=0): the residuals are then formed
+// one by one.
+static bool joint_buffers(tfm_pcg *h) {
+  if (env_int("TFM_PCG_JOINT", 1) == 0) return false;
+  if (!h->xy64 && hipMalloc(&h->xy64, 2 * sizeof(double) * (size_t)h->n * h->nrp) != hipSuccess) {
+    (void)hipGetLastError();
+    h->xy64 = nullptr;
+  }
+  return h->xy64 != nullptr;
 }
 
 static void pcg_free(tfm_pcg *h) {
@@ -2889,6 +2900,7 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
   auto residual = [&](const double *bb, const double *xx, double *res, double *rr, double *b2) -> int {
     return fem_residual(h, s, *sys, bb, xx, res, rr, b2, extended);
   };
+  auto joint = [&](int cols) { return cols > 1 && sys->val64 && !extended && joint_buffers(h); };
   h->fallback_iters = 0;
   h->path = TFM_PATH_GENERAL;
   TFM_ND_SWITCH(m.ndof, TFM_NRP_SWITCH(nrp, {
@@ -2925,10 +2937,7 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
         return spmv_launch<double, ND, NRP>(s, m, sys->val64, xi, yo);
       };
       ops.residual = residual;
-      if (sys->val64 && !extended)
-        ops.spmv64 = [&](const double *xi, double *yo) -> int {
-          return spmv_launch<double, ND, NRP>(s, m, sys->val64, xi, yo);
-        };
+      if (joint(NRP)) ops.spmv64 = ops.spmv;
       if (cs) set_coarse_ops<double, ND, NRP>(ops, s, m, *cs, sys->con, cs->inv64);
       return run_pcg<double, ND, NRP>(h, s, m.n_nod, ops, b, x, nrhs, rtol, inner_rtol,
                                       final_rtol, its, relres, out);
@@ -2950,10 +2959,10 @@ extern "C" int tfm_pcg_solve(tfm_pcg_t *h, tfm_stream_t stream, const tfm_system
           return spmv_launch<float, ND, NRP>(s, m, sys->val32, xi, yo);
         };
         ops.residual = residual;
-      if (sys->val64 && !extended)
-        ops.spmv64 = [&](const double *xi, double *yo) -> int {
-          return spmv_launch<double, ND, NRP>(s, m, sys->val64, xi, yo);
-        };
+        if (joint(NRP))
+          ops.spmv64 = [&](const double *xi, double *yo) -> int {
+            return spmv_launch<double, ND, NRP>(s, m, sys->val64, xi, yo);
+          };
         if (cs) set_coarse_ops<float, ND, NRP>(ops, s, m, *cs, sys->con, cs->inv32);
         rc = run_pcg<float, ND, NRP>(h, s, m.n_nod, ops, b, x, nrhs, rtol, inner_rtol, final_rtol,
                                      iters, relres, outer);
