@@ -131,6 +131,20 @@ __global__ void __launch_bounds__(256) k_pattern_kmap(tfm_mesh_t m, int32_t *k_m
   }
 }
 
+// The same for any number of element nodes: a block per element.
+__global__ void __launch_bounds__(256) k_pattern_kmap_any(tfm_mesh_t m, int32_t *k_map) {
+  const int64_t e = xcd_block();
+  const int npe = m.npe, nd = m.ndof, W = npe * nd;
+  for (int t = threadIdx.x; t < W * W; t += 256) {
+    const int r = t / W, c = t - r * W;
+    const int i = r / nd, a = r - i * nd, j = c / nd, b = c - j * nd;
+    const int64_t n = m.elements[e * npe + i];
+    const int len = nd * (m.adj_ptr[n + 1] - m.adj_ptr[n]);
+    const int pos = m.epos[(e * npe + i) * npe + j];
+    k_map[e * W * W + t] = (int32_t)(m.val_ptr[n] + a * len + pos * nd + b);
+  }
+}
+
 template <int ND>
 static int pattern_expand(hipStream_t s, const tfm_mesh_t &m, int64_t *rows, int64_t *cols,
                           int64_t *rowptr, int32_t *k_map, int32_t *diag_map) {
@@ -145,7 +159,7 @@ static int pattern_expand(hipStream_t s, const tfm_mesh_t &m, int64_t *rows, int
       case 4: hipLaunchKernelGGL((k_pattern_kmap<4, ND>), dim3(by4), dim3(256), 0, s, m, k_map); break;
       case 8: hipLaunchKernelGGL((k_pattern_kmap<8, ND>), dim3(by4), dim3(256), 0, s, m, k_map); break;
       case 20: hipLaunchKernelGGL((k_pattern_kmap<20, ND>), dim3(by1), dim3(256), 0, s, m, k_map); break;
-      default: TFM_REQUIRE(false, "unsupported number of element nodes");
+      default: hipLaunchKernelGGL(k_pattern_kmap_any, dim3(by1), dim3(256), 0, s, m, k_map);
     }
     TFM_CHECK_LAUNCH();
   }
@@ -1098,6 +1112,78 @@ __global__ void __launch_bounds__(64) k_assemble_elements(tfm_mesh_t m, const do
   tile_epilogue<NDOF, NW>(m, n0, acc, stride, cmask, tile, v64, v32, dblk, diff32);
 }
 
+// The same for any number of element nodes, and for degrees whose rows do not fit
+// LDS: a block per node, which gathers every entry from the node's elements.
+template <int NDOF>
+__global__ void __launch_bounds__(64) k_assemble_elements_any(tfm_mesh_t m, const double *kin,
+                                                              const uint8_t *con, double *v64,
+                                                              float *v32, double *dblk,
+                                                              int diff32) {
+  constexpr int ND2 = NDOF * NDOF;
+  extern __shared__ signed char slot_dyn[];  // [max_inc * max_deg]
+  const int64_t n = xcd_block();
+  const int tid = threadIdx.x;
+  const int npe = m.npe, W = npe * NDOF;
+  const int a0 = m.adj_ptr[n];
+  const int deg = m.adj_ptr[n + 1] - a0;
+  const int64_t vb = m.val_ptr[n];
+  if (deg == 0) {
+    if (tid < NDOF) {
+      const double v = con[n * NDOF + tid] ? 1.0 : 0.0;
+      if (v64) v64[vb + tid] = v;
+      if (v32) v32[vb + tid] = (float)v;
+    }
+    for (int t = tid; t < ND2; t += 64) {
+      const int a = t / NDOF, b = t - a * NDOF;
+      dblk[n * ND2 + t] = (a == b && con[n * NDOF + a]) ? 1.0 : 0.0;
+    }
+    return;
+  }
+  const int inc0 = m.ne_ptr[n], ninc = m.ne_ptr[n + 1] - inc0;
+  for (int t = tid; t < ninc * deg; t += 64) slot_dyn[t] = -1;
+  __syncthreads();
+  for (int t = tid; t < ninc * npe; t += 64) {
+    const int k = t / npe, j = t - k * npe;
+    const int64_t e = m.ne_elem[inc0 + k];
+    slot_dyn[k * deg + m.epos[(e * npe + m.ne_loc[inc0 + k]) * npe + j]] = (signed char)j;
+  }
+  __syncthreads();
+  int pself = 0;
+  for (int p = 0; p < deg; ++p)
+    if (m.adj[a0 + p] == n) pself = p;
+  const int L = NDOF * deg;
+  // entry (a, p, b) of the node's rows with the Dirichlet epilogue applied
+  auto entry = [&](int a, int p, int b) -> double {
+    double v = 0.0;
+    for (int k = 0; k < ninc; ++k) {
+      const int j = slot_dyn[k * deg + p];
+      if (j >= 0) {
+        const int64_t e = m.ne_elem[inc0 + k];
+        const int i = m.ne_loc[inc0 + k];
+        v += kin[e * W * W + (int64_t)(i * NDOF + a) * W + j * NDOF + b];
+      }
+    }
+    const int64_t row = n * NDOF + a;
+    const int64_t col = (int64_t)m.adj[a0 + p] * NDOF + b;
+    if (con[row] || con[col]) v = (row == col) ? 1.0 : 0.0;
+    return v;
+  };
+  for (int q = tid; q < ND2 * deg; q += 64) {
+    const int a = q / L, rem = q - a * L, p = rem / NDOF, b = rem - p * NDOF;
+    const double v = entry(a, p, b);
+    if (v64) v64[vb + q] = v;
+    if (v32 && (p != pself || !diff32)) v32[vb + q] = (float)v;
+    if (p == pself) dblk[n * ND2 + a * NDOF + b] = v;
+  }
+  // FP32 difference form: the diagonal block holds the FP64 row sums
+  if (v32 && diff32 && tid < ND2) {
+    const int a = tid / NDOF, b = tid - a * NDOF;
+    double r = 0.0;
+    for (int p = 0; p < deg; ++p) r += entry(a, p, b);
+    v32[vb + a * L + pself * NDOF + b] = (float)r;
+  }
+}
+
 // Sensitivities of lam^T K(p) u per element (see tfm_sensitivity in tfm.h):
 // a lane per Gauss point, whose geometry serves every right-hand side.
 // Hexa2 21x19x23 with 12 right-hand sides: 1385 us with a lane per node and
@@ -1327,12 +1413,22 @@ int launch_assemble_elements(hipStream_t s, const tfm_mesh_t &m, const double *k
                              const uint8_t *con, double *v64, float *v32, double *dblk,
                              bool diff32) {
   if (m.n_nod == 0) return TFM_OK;
-  TFM_REQUIRE((size_t)m.max_inc * m.max_deg <= 48 * 1024,
-              "node degree too large for the assembly kernel");
-  auto go = [&](auto kernel, int nw, int nd) -> int {
-    // at most 73 bytes per neighbour: 72 KB at the largest degree (990) that
-    // the bound above allows for 20 nodes per element
+  const size_t slots = (size_t)m.max_inc * m.max_deg;
+  TFM_REQUIRE(slots <= 48 * 1024, "node degree too large for the assembly kernel");
+  TFM_REQUIRE(m.npe <= 127, "too many element nodes for the assembly kernel");
+  auto any = [&](auto kernel) -> int {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)m.n_nod), dim3(64), slots, s, m, k, con, v64, v32,
+                       dblk, (int)diff32);
+    TFM_CHECK_LAUNCH();
+    return TFM_OK;
+  };
+  auto go = [&](auto kernel, int nw, auto general, int nd) -> int {
+    // per neighbour and node of the tile a block of values and a byte. A pattern
+    // whose max_deg follows from its max_inc needs at most 112 KB under the bound
+    // above (Tetra1, three DOFs, four nodes: 292 bytes times 384); a caller may
+    // state a larger max_deg.
     const size_t shm = (sizeof(double) * nd * nd + 1) * nw * (size_t)m.max_deg;
+    if (shm > 128 * 1024) return any(general);
     if (shm > 60 * 1024)
       TFM_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
@@ -1341,20 +1437,21 @@ int launch_assemble_elements(hipStream_t s, const tfm_mesh_t &m, const double *k
     TFM_CHECK_LAUNCH();
     return TFM_OK;
   };
-  auto by_ndof = [&](auto npe) -> int {
-    constexpr int N = decltype(npe)::value;
-    switch (m.ndof) {
-      case 1: return go(&k_assemble_elements<N, 1>, 64 / assemble_lanes(N, 1), 1);
-      case 2: return go(&k_assemble_elements<N, 2>, 64 / assemble_lanes(N, 2), 2);
-      case 3: return go(&k_assemble_elements<N, 3>, 64 / assemble_lanes(N, 3), 3);
-      default: TFM_REQUIRE(false, "ndof must be 1, 2 or 3");
+  auto by_npe = [&](auto ndof) -> int {
+    constexpr int ND = decltype(ndof)::value;
+    auto general = &k_assemble_elements_any<ND>;
+    switch (m.npe) {
+      case 4: return go(&k_assemble_elements<4, ND>, 64 / assemble_lanes(4, ND), general, ND);
+      case 8: return go(&k_assemble_elements<8, ND>, 64 / assemble_lanes(8, ND), general, ND);
+      case 20: return go(&k_assemble_elements<20, ND>, 64 / assemble_lanes(20, ND), general, ND);
+      default: return any(general);
     }
   };
-  switch (m.npe) {
-    case 4: return by_ndof(std::integral_constant<int, 4>{});
-    case 8: return by_ndof(std::integral_constant<int, 8>{});
-    case 20: return by_ndof(std::integral_constant<int, 20>{});
-    default: TFM_REQUIRE(false, "unsupported number of element nodes");
+  switch (m.ndof) {
+    case 1: return by_npe(std::integral_constant<int, 1>{});
+    case 2: return by_npe(std::integral_constant<int, 2>{});
+    case 3: return by_npe(std::integral_constant<int, 3>{});
+    default: TFM_REQUIRE(false, "ndof must be 1, 2 or 3");
   }
 }
 
