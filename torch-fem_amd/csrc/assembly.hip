@@ -1184,16 +1184,27 @@ __global__ void __launch_bounds__(64) k_assemble_elements_any(tfm_mesh_t m, cons
   }
 }
 
+// Elements per block of the sensitivities: fewer where a lane would have an
+// element of its own and the layout is general. The outputs (82 values of an
+// anisotropic Tetra1) are the work then, and 64 elements' of them one after the
+// other leave a small mesh to a few waves and five waves to a CU. Anisotropic
+// Tetra1, 16 right-hand sides: 750 elements 207 us with 64 to a block, 61 with 8
+// and 84 with 16 (a lane per node 72); 93,750 elements 647, 481 and 380 (561); the
+// line between 8 and 16 lies at a block of 16 for every CU, four times over.
+template <class E, int MAT> constexpr bool sens_outputs() {
+  return E::NGP == 1 && (MAT == TFM_MAT_GENERAL || MAT == TFM_MAT_HEAT_GENERAL);
+}
+
 // Sensitivities of lam^T K(p) u per element (see tfm_sensitivity in tfm.h):
 // a lane per Gauss point, whose geometry serves every right-hand side.
 // Hexa2 21x19x23 with 12 right-hand sides: 1385 us with a lane per node and
 // the geometry formed for each, now 80; Hexa1 47x41x52 with one 186 us, now 28.
-template <class E, int NDOF, int MAT>
+template <class E, int NDOF, int MAT, int EPB>
 __global__ void __launch_bounds__(64) k_sensitivity(tfm_mesh_t m, tfm_material_t mat,
                                                     const double *u, const double *lam,
                                                     int nrhs, double sign, double *out) {
   constexpr int NPE = E::NPE, NGP = E::NGP, D = E::DIM, NP = mat_nparam(MAT, D);
-  constexpr int EPB = point_elems<E>(), NQ = NDOF * D;
+  constexpr int NQ = NDOF * D;
   constexpr bool ISO = (MAT == TFM_MAT_ISO || MAT == TFM_MAT_HEAT_ISO);
   constexpr int NI = MAT == TFM_MAT_ISO ? 2 : 1, NO = (ISO ? NI : NP) + 1;
   __shared__ double tbl[NGP][odd(D * NPE)];
@@ -1202,7 +1213,7 @@ __global__ void __launch_bounds__(64) k_sensitivity(tfm_mesh_t m, tfm_material_t
   using Params = PointParams<E, MAT>;
   __shared__ double MP[Params::ROWS][Params::STRIDE];
   // general layouts: w detJ s grad(lam), sym(grad u) or grad u, and the energy
-  __shared__ double st[ISO ? 1 : 64][odd(2 * NQ + 1)];
+  __shared__ double st[ISO ? 1 : EPB * NGP][odd(2 * NQ + 1)];
   const int lane = threadIdx.x, el = lane / NGP, g = lane % NGP;
   const int64_t e0 = xcd_block() * EPB;
   const int ne = (int)(m.n_elem - e0 < EPB ? m.n_elem - e0 : EPB);
@@ -1473,10 +1484,18 @@ int launch_sensitivity(hipStream_t s, const tfm_mesh_t &m, const tfm_material_t 
                        const double *u, const double *lam, int nrhs, double sign, double *out) {
   if (m.n_elem == 0 || nrhs == 0) return TFM_OK;
   TFM_DISPATCH_ALL(m, mat, {
-    constexpr int EPB = point_elems<ET>();
-    const unsigned nb = (unsigned)((m.n_elem + EPB - 1) / EPB);
-    hipLaunchKernelGGL((k_sensitivity<ET, ND, MK>), dim3(nb), dim3(64), 0, s, m, mat, u, lam,
-                       nrhs, sign, out);
+    auto go = [&](auto elems) {
+      constexpr int EPB = decltype(elems)::value;
+      const unsigned nb = (unsigned)((m.n_elem + EPB - 1) / EPB);
+      hipLaunchKernelGGL((k_sensitivity<ET, ND, MK, EPB>), dim3(nb), dim3(64), 0, s, m, mat, u,
+                         lam, nrhs, sign, out);
+    };
+    if constexpr (sens_outputs<ET, MK>()) {
+      if (m.n_elem <= 4 * 256 * 16) go(std::integral_constant<int, 8>{});
+      else go(std::integral_constant<int, 16>{});
+    } else {
+      go(std::integral_constant<int, point_elems<ET>()>{});
+    }
     TFM_CHECK_LAUNCH();
   });
   return TFM_OK;
