@@ -337,6 +337,92 @@ __global__ void __launch_bounds__(64 * PNB) k_adj_fill(const int32_t *el, int np
   }
 }
 
+// ------------------------------------- adjacency, a thread per node
+// For large meshes whose nodes have few candidates: a wave's sort is then half
+// empty or emptier. The whole pattern with a thread and with a wave per node, us:
+// Quad1 (16 candidates) 600 x 601 384 and 572, 300 x 301 236 and 305, 100 x 101 204
+// and 216, 60 x 61 206 and 198; Hexa1 300 x 300 x 1 (32) 356 and 408, 200 x 200 x 2
+// (42) 434 and 351.
+bool few_candidates(int64_t n_elem, int npe, int64_t n_nod) {
+  return n_nod >= 8192 && n_elem * npe * npe <= 32 * n_nod;
+}
+
+// The set of node_union by insertion with binary search in a list of at most
+// PMAXDEG entries. Returns its size, -1 on overflow.
+__device__ int node_union_thread(const int32_t *el, int npe, const int32_t *inc, int ninc,
+                                 int32_t *lst) {
+  int deg = 0;
+  for (int k = 0; k < ninc; ++k) {
+    const int32_t *en = el + (int64_t)inc[k] * npe;
+    for (int j = 0; j < npe; ++j) {
+      const int32_t c = en[j];
+      int lo = 0, hi = deg;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (lst[mid] < c) lo = mid + 1;
+        else hi = mid;
+      }
+      if (lo < deg && lst[lo] == c) continue;
+      if (deg == PMAXDEG) return -1;
+      for (int q = deg; q > lo; --q) lst[q] = lst[q - 1];
+      lst[lo] = c;
+      ++deg;
+    }
+  }
+  return deg;
+}
+
+__global__ void k_adj_count_thread(const int32_t *el, int npe, int64_t n_nod,
+                                   const int32_t *ne_ptr, const int32_t *ne_elem, int ndof,
+                                   int32_t *deg, int32_t *nval, int32_t *max_deg, int32_t *bad) {
+  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= n_nod) return;
+  int32_t lst[PMAXDEG];
+  const int32_t i0 = ne_ptr[n];
+  const int d = node_union_thread(el, npe, ne_elem + i0, ne_ptr[n + 1] - i0, lst);
+  if (d < 0) *bad = 2;
+  deg[n] = d > 0 ? d : 0;
+  nval[n] = d > 0 ? d * ndof * ndof : ndof;
+  raise(max_deg, d);
+}
+
+__global__ void k_adj_fill_thread(const int32_t *el, int npe, int64_t n_nod,
+                                  const int32_t *ne_ptr, const int32_t *ne_elem,
+                                  const int32_t *adj_ptr, int32_t *adj, int16_t *adj16,
+                                  int32_t *wide) {
+  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= n_nod) return;
+  int32_t lst[PMAXDEG];
+  const int32_t i0 = ne_ptr[n], a0 = adj_ptr[n];
+  const int d = node_union_thread(el, npe, ne_elem + i0, ne_ptr[n + 1] - i0, lst);
+  for (int q = 0; q < d; ++q) {
+    adj[a0 + q] = lst[q];
+    if (adj16) {
+      const int64_t delta = (int64_t)lst[q] - n;
+      if (delta < -32768 || delta > 32767) *wide = 1;
+      adj16[a0 + q] = (int16_t)delta;
+    }
+  }
+}
+
+// epos[e][i][j]: position of element node j in the adjacency of node i
+__global__ void k_epos(const int32_t *el, int64_t n_elem, int npe, const int32_t *adj_ptr,
+                       const int32_t *adj, uint16_t *epos) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n_elem * npe * npe) return;
+  const int64_t e = t / (npe * npe);
+  const int r = (int)(t - e * npe * npe), i = r / npe, j = r - i * npe;
+  const int32_t ni = el[e * npe + i], nj = el[e * npe + j];
+  int lo = adj_ptr[ni], hi = adj_ptr[ni + 1];
+  const int base = lo;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (adj[mid] < nj) lo = mid + 1;
+    else hi = mid;
+  }
+  epos[t] = (uint16_t)(lo - base);
+}
+
 }  // namespace
 }  // namespace tfm
 
@@ -374,10 +460,14 @@ extern "C" int tfm_pattern_device_count(tfm_stream_t stream, const int32_t *elem
     hipLaunchKernelGGL(k_inc_sort, dim3(pblocks(n_nod)), dim3(PB), 0, s, n_nod,
                        (const int32_t *)ne_ptr, ne_elem, ne_loc, flags + 1);
     TFM_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_adj_count, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s,
-                       elements, (int)npe, n_nod, (const int32_t *)ne_ptr,
-                       (const int32_t *)ne_elem, (int)ndof, cnt, nval,
-                       flags + 2, flags);
+    if (few_candidates(n_elem, npe, n_nod))
+      hipLaunchKernelGGL(k_adj_count_thread, dim3(pblocks(n_nod, 64)), dim3(64), 0, s, elements,
+                         (int)npe, n_nod, (const int32_t *)ne_ptr, (const int32_t *)ne_elem,
+                         (int)ndof, cnt, nval, flags + 2, flags);
+    else
+      hipLaunchKernelGGL(k_adj_count, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s, elements,
+                         (int)npe, n_nod, (const int32_t *)ne_ptr, (const int32_t *)ne_elem,
+                         (int)ndof, cnt, nval, flags + 2, flags);
     TFM_CHECK_LAUNCH();
   }
   rc = pscan<int32_t>(s, cnt, n_nod, bsum32, adj_ptr);
@@ -408,10 +498,19 @@ extern "C" int tfm_pattern_device_fill(tfm_stream_t stream, const int32_t *eleme
   TFM_REQUIRE(ne_ptr && adj_ptr && work && adj16_fits, "null argument");
   hipStream_t s = (hipStream_t)stream;
   TFM_CHECK_HIP(hipMemsetAsync(work, 0, sizeof(int32_t), s));
-  if (n_nod > 0) {
-    hipLaunchKernelGGL(k_adj_fill, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s,
-                       elements, (int)npe, n_nod, ne_ptr,
-                       ne_elem, adj_ptr, adj, adj16, work, epos);
+  if (few_candidates(n_elem, npe, n_nod)) {
+    hipLaunchKernelGGL(k_adj_fill_thread, dim3(pblocks(n_nod, 64)), dim3(64), 0, s, elements,
+                       (int)npe, n_nod, ne_ptr, ne_elem, adj_ptr, adj, adj16, work);
+    TFM_CHECK_LAUNCH();
+    const int64_t ne = n_elem * npe * npe;
+    if (ne > 0) {
+      hipLaunchKernelGGL(k_epos, dim3(pblocks(ne)), dim3(PB), 0, s, elements, n_elem, (int)npe,
+                         adj_ptr, (const int32_t *)adj, epos);
+      TFM_CHECK_LAUNCH();
+    }
+  } else if (n_nod > 0) {
+    hipLaunchKernelGGL(k_adj_fill, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s, elements,
+                       (int)npe, n_nod, ne_ptr, ne_elem, adj_ptr, adj, adj16, work, epos);
     TFM_CHECK_LAUNCH();
   }
   int32_t wide = 0;
