@@ -163,11 +163,10 @@ __global__ void k_inc_sort(int64_t n_nod, const int32_t *ptr, int32_t *ne_elem, 
 // into a sorted list per thread, in scratch memory, took 290 us per pass on
 // 53x47x58 Hexa1 and 400 us on 13x15x11 Hexa2; this takes 89 and 29,
 // bound by the vector instructions of the sort. Filling needs 102 and 34 with epos
-// (357 and 410 before, with a search of adj in memory for every pair).
+// (357 and 410 before, with a search of adj in memory for every pair). A block is
+// one wave: four of them took 84 and 106 us (one: 89 and 102) on Hexa1, 46 and 35
+// (29 and 34) on Hexa2, where few nodes have the long lists.
 constexpr int PROOM = 256;  // values that one sort holds
-// nodes (waves) per block: four took 84 and 106 us (one: 89 and 102) on Hexa1,
-// 46 and 35 (29 and 34) on Hexa2, where few nodes have the long lists
-constexpr int PNB = 1;
 constexpr int32_t PNONE = 0x7fffffff;
 
 // LDS accesses of a wave complete in order; the compiler must keep them so.
@@ -203,7 +202,7 @@ template <int J> __device__ __forceinline__ int32_t partner_min_max(int32_t v, b
 // One step of the network over R registers: the partners at distance J in
 // runs of K sorted alternately up and down.
 template <int R, int K, int J> __device__ __forceinline__ void sort_step(int32_t (&v)[R]) {
-  const int lane = threadIdx.x % 64;
+  const int lane = threadIdx.x;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int i = r * 64 + lane;
@@ -229,7 +228,7 @@ template <int R> __device__ __forceinline__ void wave_sort(int32_t (&v)[R]) {
 
 // Sorts v and puts its distinct values (PNONE apart) into lst; their number.
 template <int R> __device__ __forceinline__ int sort_distinct(int32_t (&v)[R], int32_t *lst) {
-  const int lane = threadIdx.x % 64;
+  const int lane = threadIdx.x;
   wave_sort<R>(v);
   int n = 0;
   int32_t before = PNONE;  // the last value of the registers before
@@ -250,7 +249,7 @@ template <int R> __device__ __forceinline__ int sort_distinct(int32_t (&v)[R], i
 // when it belongs to an element) in lst[PROOM]; its size, -1 beyond PMAXDEG.
 __device__ __forceinline__ int node_union(const int32_t *el, int npe, const int32_t *inc,
                                           int ninc, int32_t *lst) {
-  const int lane = threadIdx.x % 64, C = ninc * npe;
+  const int lane = threadIdx.x, C = ninc * npe;
   auto candidate = [&](int i) -> int32_t {
     return i < C ? el[(int64_t)inc[i / npe] * npe + i % npe] : PNONE;
   };
@@ -283,17 +282,15 @@ __device__ __forceinline__ int node_union(const int32_t *el, int npe, const int3
 
 // deg[n] and the value count of n's rows (deg * ndof^2, or ndof for a node
 // of no element)
-__global__ void __launch_bounds__(64 * PNB) k_adj_count(const int32_t *el, int npe,
-                                                  int64_t n_nod, const int32_t *ne_ptr,
-                                                  const int32_t *ne_elem, int ndof, int32_t *deg, int32_t *nval,
+__global__ void __launch_bounds__(64) k_adj_count(const int32_t *el, int npe,
+                                                  const int32_t *ne_ptr, const int32_t *ne_elem,
+                                                  int ndof, int32_t *deg, int32_t *nval,
                                                   int32_t *max_deg, int32_t *bad) {
-  __shared__ int32_t lists[PNB][PROOM];
-  int32_t *lst = lists[threadIdx.x / 64];
-  const int64_t n = xcd_block() * PNB + threadIdx.x / 64;
-  if (n >= n_nod) return;
+  __shared__ int32_t lst[PROOM];
+  const int64_t n = xcd_block();
   const int32_t i0 = ne_ptr[n];
   const int d = node_union(el, npe, ne_elem + i0, ne_ptr[n + 1] - i0, lst);
-  if (threadIdx.x % 64 != 0) return;
+  if (threadIdx.x != 0) return;
   if (d < 0) *bad = 2;
   deg[n] = d > 0 ? d : 0;
   nval[n] = d > 0 ? d * ndof * ndof : ndof;
@@ -303,15 +300,13 @@ __global__ void __launch_bounds__(64 * PNB) k_adj_count(const int32_t *el, int n
 // adj (and the 16-bit offsets adj - n when adj16 is given; *wide is set if
 // some offset does not fit), and epos[e][i][j], the position of element node j
 // in the adjacency of node i, for the incidences (e, i) of the node
-__global__ void __launch_bounds__(64 * PNB) k_adj_fill(const int32_t *el, int npe,
-                                                 int64_t n_nod, const int32_t *ne_ptr,
-                                                 const int32_t *ne_elem, const int32_t *adj_ptr, int32_t *adj,
+__global__ void __launch_bounds__(64) k_adj_fill(const int32_t *el, int npe,
+                                                 const int32_t *ne_ptr, const int32_t *ne_elem,
+                                                 const int32_t *adj_ptr, int32_t *adj,
                                                  int16_t *adj16, int32_t *wide, uint16_t *epos) {
-  __shared__ int32_t lists[PNB][PROOM];
-  int32_t *lst = lists[threadIdx.x / 64];
-  const int lane = threadIdx.x % 64;
-  const int64_t n = xcd_block() * PNB + threadIdx.x / 64;
-  if (n >= n_nod) return;
+  __shared__ int32_t lst[PROOM];
+  const int lane = threadIdx.x;
+  const int64_t n = xcd_block();
   const int32_t i0 = ne_ptr[n], ninc = ne_ptr[n + 1] - i0, a0 = adj_ptr[n];
   const int d = node_union(el, npe, ne_elem + i0, ninc, lst);
   for (int q = lane; q < d; q += 64) {
@@ -465,9 +460,9 @@ extern "C" int tfm_pattern_device_count(tfm_stream_t stream, const int32_t *elem
                          (int)npe, n_nod, (const int32_t *)ne_ptr, (const int32_t *)ne_elem,
                          (int)ndof, cnt, nval, flags + 2, flags);
     else
-      hipLaunchKernelGGL(k_adj_count, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s, elements,
-                         (int)npe, n_nod, (const int32_t *)ne_ptr, (const int32_t *)ne_elem,
-                         (int)ndof, cnt, nval, flags + 2, flags);
+      hipLaunchKernelGGL(k_adj_count, dim3((unsigned)n_nod), dim3(64), 0, s, elements, (int)npe,
+                         (const int32_t *)ne_ptr, (const int32_t *)ne_elem, (int)ndof, cnt, nval,
+                         flags + 2, flags);
     TFM_CHECK_LAUNCH();
   }
   rc = pscan<int32_t>(s, cnt, n_nod, bsum32, adj_ptr);
@@ -509,8 +504,8 @@ extern "C" int tfm_pattern_device_fill(tfm_stream_t stream, const int32_t *eleme
       TFM_CHECK_LAUNCH();
     }
   } else if (n_nod > 0) {
-    hipLaunchKernelGGL(k_adj_fill, dim3(pblocks(n_nod, PNB)), dim3(64 * PNB), 0, s, elements,
-                       (int)npe, n_nod, ne_ptr, ne_elem, adj_ptr, adj, adj16, work, epos);
+    hipLaunchKernelGGL(k_adj_fill, dim3((unsigned)n_nod), dim3(64), 0, s, elements, (int)npe,
+                       ne_ptr, ne_elem, adj_ptr, adj, adj16, work, epos);
     TFM_CHECK_LAUNCH();
   }
   int32_t wide = 0;
