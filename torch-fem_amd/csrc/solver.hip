@@ -1335,8 +1335,8 @@ static SpmvShape spmv_shape(const tfm_mesh_t &m, int nrp) {
   // FP64 with one or two rhs: the full grid (one node per team); with more,
   // a capped grid-stride grid, so that the one-block scalar kernel sums few
   // partial sets (35k blocks x 16 rhs of Hexa2 32^3 took it 84 us). FP32
-  // with 16 rhs on Hexa2 32^3: 1024 blocks ran the step in 1,015 ms against
-  // 1,065 ms with 512
+  // with 16 rhs on Hexa2 32^3: a step on 1024 blocks 998 ms, on 512 1,287, on
+  // 2048 1,013; the plain product on 1024 144 us, on 512 156
   sh.cap = fp64 ? (nrp >= 4 ? RBA / 2 : (1 << 30)) : (nrp <= 2 ? RBA : RBA / 2);
   static const int g_env = env_int("TFM_SPMV_GRID", 0);
   static const int f_env = env_int("TFM_SPMV_SCAL", -1);
@@ -1386,11 +1386,8 @@ static SpmvShape spmv_shape(const tfm_mesh_t &m, int nrp) {
 template <typename T, int ND, int NRP>
 static int spmv_launch(hipStream_t s, const tfm_mesh_t &m, const T *val, const T *x, T *y) {
   const SpmvShape sh = spmv_shape<T>(m, NRP);
-  // the plain FP32 product with 16 rhs ran faster on 512 blocks (178 us)
-  // than on the fused product's 1024 (204 us), on Hexa2 32^3
-  const int cap = sizeof(T) == 4 && NRP > 8 ? std::min(sh.cap, RBA / 4) : sh.cap;
   TFM_TEAM_SWITCH(sh.tl, {
-    const unsigned g = grid_for(m.n_nod, BS / TL, cap);
+    const unsigned g = grid_for(m.n_nod, BS / TL, sh.cap);
     if (m.adj16)
       hipLaunchKernelGGL((k_spmv<T, ND, TL, NRP, true>), dim3(g), dim3(BS), 0, s, m, val, x, y);
     else
@@ -1563,6 +1560,9 @@ template <int ND, int NRP> struct CoarseShape {
   static constexpr int THREADS = NRP >= 4 ? 1024 : 256;
   static constexpr int WAVES = THREADS / 64;
   static constexpr int AGGS = ND == 1 && NRP <= 2 ? 4 : 1;  // per block of the coarse product
+  // Beyond about 260,000 nodes the aggregates no longer grow in number and the
+  // threads loop over their chunk: 96^3 Hexa1 (913,000 nodes) 31.7 us for the
+  // update (3.8 TB/s) and 23.5 for the coarse product, beside 194 for A.
   static int chunks(int64_t n_nod, int n_agg) {
     const int64_t per = (n_nod + n_agg - 1) / n_agg;
     if (AGGS > 1) return 1;
