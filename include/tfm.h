@@ -190,7 +190,7 @@ int tfm_pattern_device_fill(tfm_stream_t s, const int32_t *elements, int64_t n_e
 /* The reference's index arrays on the device: glob_idx rows/cols (int64,
  * base.py:112-117), CSR row pointer, k_map (int32 [n_elem*(npe*ndof)^2],
  * base.py:94-104) and diag_map (int32 [n_dofs], base.py:106-108).
- * Any output pointer may be NULL. */
+ * Any output pointer may be NULL; any number of nodes per element. */
 int tfm_pattern_expand(tfm_stream_t s, const tfm_mesh_t *m, int64_t *rows,
                        int64_t *cols, int64_t *rowptr, int32_t *k_map,
                        int32_t *diag_map);
@@ -234,7 +234,8 @@ int tfm_assemble(tfm_stream_t s, const tfm_mesh_t *m, const tfm_material_t *mat,
 
 /* Same Dirichlet epilogue and outputs as tfm_assemble, from caller-supplied
  * element matrices k [n_elem, npe*ndof, npe*ndof] (FEM.assemble_matrix,
- * base.py:398-426, as an ordered gather instead of index_add_). */
+ * base.py:398-426, as an ordered gather instead of index_add_), of at most 127
+ * nodes per element and max_inc * max_deg <= 48 K. */
 int tfm_assemble_elements(tfm_stream_t s, const tfm_mesh_t *m, const double *k,
                           const uint8_t *con, double *val64, float *val32,
                           double *diag_blocks, int32_t fp32_form);
@@ -298,7 +299,9 @@ int tfm_csr_spmv(tfm_stream_t s, int64_t n, const int64_t *rowptr,
 
 /* ------------------------------------------------------------ PCG solver */
 /* Workspace handle for up to nrhs simultaneous right-hand sides of size n
- * (like the reference's AmgXSolver handle, amgx.py:211-395). */
+ * (like the reference's AmgXSolver handle, amgx.py:211-395): five vectors of
+ * n x nrhs (nrhs rounded up to a power of two) in FP64, and two more from the
+ * first solve that refines several right-hand sides together. */
 int tfm_pcg_create(tfm_pcg_t **h, int64_t n, int32_t nrhs, int32_t max_iter);
 int tfm_pcg_destroy(tfm_pcg_t *h);
 
