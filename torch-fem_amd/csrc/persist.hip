@@ -779,11 +779,11 @@ int persist_solve(hipStream_t s, const PersistJob &J, PersistResult *res, bool *
   const int nd = csr ? 1 : J.m->ndof;
   const int64_t n_nod = csr ? J.n : J.m->n_nod;
   if (n_nod < 1 || J.val64 == nullptr || nd < 1 || nd > 3) return TFM_OK;
-  int dev = 0, cus = 0, lds = 0;
-  TFM_CHECK_HIP(hipGetDevice(&dev));
+  const int dev = J.device;
+  int cus = 0, lds = 0;
   TFM_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   TFM_CHECK_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-  if (dev >= 64 || lds < 160 * 1024) return TFM_OK;
+  if (dev < 0 || dev >= 64 || lds < 160 * 1024) return TFM_OK;
   if (std::chrono::steady_clock::now() < g_rest[dev]) return TFM_OK;
   const int max_blocks = std::min(cus, PERSIST_MAX_BLOCKS);
   const unsigned size = J.fp64 ? 8u : 4u;

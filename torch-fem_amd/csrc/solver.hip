@@ -2151,10 +2151,14 @@ static int pcg_alloc(tfm_pcg *h) {
 // one by one.
 static bool joint_buffers(tfm_pcg *h) {
   if (env_int("TFM_PCG_JOINT", 1) == 0) return false;
-  if (!h->xy64 && hipMalloc(&h->xy64, 2 * sizeof(double) * (size_t)h->n * h->nrp) != hipSuccess) {
+  if (h->xy64) return true;
+  int current = 0;  // the caller's device need not be the handle's
+  if (hipGetDevice(&current) != hipSuccess || hipSetDevice(h->device) != hipSuccess) return false;
+  if (hipMalloc(&h->xy64, 2 * sizeof(double) * (size_t)h->n * h->nrp) != hipSuccess) {
     (void)hipGetLastError();
     h->xy64 = nullptr;
   }
+  (void)hipSetDevice(current);
   return h->xy64 != nullptr;
 }
 
@@ -2774,6 +2778,7 @@ bool try_persist(tfm_pcg *h, hipStream_t s, PersistJob &job, int32_t *iters, dou
                  int32_t *outer, int *rc) {
   h->path = TFM_PATH_GENERAL;
   if (h->timing || (job.m && job.m->nnz == h->no_fit[job.fp64])) return false;
+  job.device = h->device;
   job.u = h->u;
   job.p = h->p;
   job.scratch = h->persist;

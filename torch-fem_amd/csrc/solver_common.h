@@ -149,7 +149,8 @@ constexpr size_t PERSIST_SCRATCH_BYTES =
 struct PersistJob {
   // rows: the node blocks of a mesh, or a general CSR matrix (m == nullptr)
   const tfm_mesh_t *m = nullptr;
-  int64_t n = 0;  // rows of the CSR matrix
+  int64_t n = 0;   // rows of the CSR matrix
+  int device = 0;  // of the stream and the buffers
   const int64_t *rowptr = nullptr;
   const int32_t *col = nullptr;
   bool fp64 = true;
